@@ -719,18 +719,51 @@ __global__ __launch_bounds__(kThreads) void rabitq_encode_kernel(const float* xr
 // a block); the blocks' partial sums are then added in block order.
 constexpr uint32_t kColBlock = 4096;
 
-template <class T>
-__global__ __launch_bounds__(kThreads) void col_partial_kernel(const T* rows, uint32_t dim,
-                                                               uint64_t n, double* partial)
+// Each thread owns kV neighbouring columns of one block of rows and adds them
+// row by row; kColBatch rows are loaded before the first is added, because a
+// chain of one load per add is bound by memory latency (150,000 x 512 f16 in
+// six label groups: 13.9 ms with one column slab a workgroup and one load in
+// flight, 0.55 ms here).  Grid: (row blocks, column slabs of 64 kV).
+constexpr int kColBatch = 32;
+
+template <class T, int kV>
+struct alignas(sizeof(T) * kV) Pack {
+    T v[kV];
+};
+
+template <class T, int kV>
+__global__ __launch_bounds__(kWave) void col_partial_kernel(const T* rows, uint32_t dim,
+                                                            uint64_t n, double* partial)
 {
+    using P = Pack<T, kV>;
     const uint64_t b = blockIdx.x;
     const uint64_t s = b * kColBlock;
     const uint64_t e = s + kColBlock < n ? s + kColBlock : n;
-    for (uint32_t d = threadIdx.x; d < dim; d += kThreads) {
-        double sum = 0.0;
-        for (uint64_t i = s; i < e; ++i) sum += static_cast<double>(to_f(rows[i * dim + d]));
-        partial[b * dim + d] = sum;
+    const uint32_t d = (blockIdx.y * kWave + threadIdx.x) * kV;
+    if (d >= dim) return;  // dim is a multiple of kV
+    const T* p = rows + s * dim + d;
+    double sum[kV];
+#pragma unroll
+    for (int v = 0; v < kV; ++v) sum[v] = 0.0;
+    uint64_t i = s;
+    for (; i + kColBatch <= e; i += kColBatch) {
+        P x[kColBatch];
+#pragma unroll
+        for (int t = 0; t < kColBatch; ++t)
+            x[t] = *reinterpret_cast<const P*>(p + static_cast<size_t>(t) * dim);
+        p += static_cast<size_t>(kColBatch) * dim;
+#pragma unroll
+        for (int t = 0; t < kColBatch; ++t)
+#pragma unroll
+            for (int v = 0; v < kV; ++v) sum[v] += static_cast<double>(to_f(x[t].v[v]));
     }
+    for (; i < e; ++i, p += dim) {
+        const P x = *reinterpret_cast<const P*>(p);
+#pragma unroll
+        for (int v = 0; v < kV; ++v) sum[v] += static_cast<double>(to_f(x.v[v]));
+    }
+#pragma unroll
+    for (int v = 0; v < kV; ++v) partial[b * dim + d + v] = sum[v];
 }
 
 __global__ void col_mean_kernel(const double* partial, uint32_t dim, uint64_t blocks, uint64_t n,
@@ -741,6 +774,107 @@ __global__ void col_mean_kernel(const double* partial, uint32_t dim, uint64_t bl
     double sum = 0.0;
     for (uint64_t b = 0; b < blocks; ++b) sum += partial[b * dim + d];
     mean[d] = sum / static_cast<double>(n);
+}
+
+// A chain over the dims of each of 64 rows, one row per lane, the rows read
+// whole lines at a time: 128 bytes of every row are loaded by eight lanes (16
+// bytes each) into a [64][33]-word LDS tile of the wave (the odd stride keeps
+// the per-row reads free of bank conflicts), the next 128 bytes are requested,
+// and each lane then takes its own row's elements from LDS, four at a time in
+// order: f(d, v) gets elements d .. d + 3.  Needs rows of whole 16-byte
+// vectors (so dim is a multiple of 4).  With a lane reading its own row from
+// memory a wave's load touches 64 lines for 64 elements.
+constexpr int kRowTileWords = 33 * kWave;
+
+template <class T>
+__device__ __forceinline__ void unpack4(const uint32_t* w, float (&v)[4])
+{
+    constexpr int kWords = static_cast<int>(sizeof(T));
+    uint32_t u[kWords];
+#pragma unroll
+    for (int i = 0; i < kWords; ++i) u[i] = w[i];
+    T t[4];
+    __builtin_memcpy(t, u, sizeof(t));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = to_f(t[i]);
+}
+
+template <class T, class F>
+__device__ __forceinline__ void tiled_row_chain(const T* rows, uint32_t dim, uint64_t r0,
+                                                uint64_t n, uint32_t* tile, int lane, F&& f)
+{
+    const uint32_t row_bytes = dim * static_cast<uint32_t>(sizeof(T));
+    constexpr uint32_t kStep = 128;  // bytes of a row per tile
+    const int sub = lane >> 3;
+    const uint32_t col = static_cast<uint32_t>(lane & 7) * 16u;
+    uint4 x[8];
+    const auto load = [&](uint32_t b0) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const uint64_t r = r0 + static_cast<uint64_t>(k * 8 + sub);
+            x[k] = r < n && b0 + col < row_bytes
+                       ? *reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(rows) +
+                                                         r * row_bytes + b0 + col)
+                       : make_uint4(0, 0, 0, 0);
+        }
+    };
+    load(0);
+    for (uint32_t b0 = 0; b0 < row_bytes; b0 += kStep) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            uint32_t* dst = tile + (k * 8 + sub) * 33 + (lane & 7) * 4;
+            dst[0] = x[k].x;
+            dst[1] = x[k].y;
+            dst[2] = x[k].z;
+            dst[3] = x[k].w;
+        }
+        __threadfence_block();
+        __builtin_amdgcn_wave_barrier();
+        if (b0 + kStep < row_bytes) load(b0 + kStep);
+        const uint32_t left = row_bytes - b0 < kStep ? row_bytes - b0 : kStep;
+        const uint32_t d0 = b0 / static_cast<uint32_t>(sizeof(T));
+        const uint32_t* mine = tile + lane * 33;
+        const uint32_t groups = left / (4u * static_cast<uint32_t>(sizeof(T)));
+        for (uint32_t g = 0; g < groups; ++g) {
+            float v[4];
+            unpack4<T>(mine + g * sizeof(T), v);
+            f(d0 + 4u * g, v);
+        }
+        __threadfence_block();
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// Whether tiled_row_chain can read `rows`.
+bool row_vectors(const void* rows, size_t row_bytes)
+{
+    return row_bytes % 16 == 0 && (reinterpret_cast<uintptr_t>(rows) & 15u) == 0;
+}
+
+// mean_dist_kernel below for rows of whole 16-byte vectors: the same chain,
+// through the tile (50,000 x 512 f16: 86 us a launch with a thread reading its
+// own row, 31 us).
+template <class T>
+__global__ __launch_bounds__(kThreads) void mean_dist_tiled_kernel(const T* rows, uint32_t dim,
+                                                                   uint64_t n, const double* mean,
+                                                                   double* dist)
+{
+    __shared__ uint32_t tiles[(kThreads / kWave) * kRowTileWords];
+    const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+    const int wave = static_cast<int>(threadIdx.x) / kWave;
+    const uint64_t r0 = static_cast<uint64_t>(blockIdx.x) * kThreads + static_cast<uint64_t>(wave) * kWave;
+    if (r0 >= n) return;
+    double s = 0.0;
+    tiled_row_chain(rows, dim, r0, n, tiles + wave * kRowTileWords, lane,
+                    [&](uint32_t d, const float (&v)[4]) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const double t = static_cast<double>(v[i]) - mean[d + i];
+                            s = fma(t, t, s);
+                        }
+                    });
+    const uint64_t r = r0 + static_cast<uint64_t>(lane);
+    if (r < n) dist[r] = s;
 }
 
 // fp64 distance of each row to the mean: sum_d (x_d - mu_d)^2, fma over d
@@ -1547,6 +1681,39 @@ int build_rabitq_encode(Context* ctx, const float* rotated, uint32_t n, uint32_t
     return GOFANN_OK;
 }
 
+namespace {
+template <class T, int kV>
+void col_partial_launch(Context* ctx, const T* rows, uint32_t dim, uint64_t n, uint64_t cblocks,
+                        double* partial)
+{
+    const dim3 grid(static_cast<uint32_t>(cblocks), (dim + kWave * kV - 1) / (kWave * kV));
+    hipLaunchKernelGGL((col_partial_kernel<T, kV>), grid, dim3(kWave), 0, ctx->stream, rows, dim, n,
+                       partial);
+}
+
+// The rows' fp64 mean, then every row's distance to it.
+template <class T>
+void medoid_dists(Context* ctx, const T* rows, uint32_t dim, uint64_t n, uint64_t cblocks,
+                  double* partial, double* mean, double* dist)
+{
+    // a 4-byte load of neighbouring columns where every row allows it
+    constexpr int kV = 4 / static_cast<int>(sizeof(T));
+    if (dim % kV == 0 && (reinterpret_cast<uintptr_t>(rows) & 3u) == 0)
+        col_partial_launch<T, kV>(ctx, rows, dim, n, cblocks, partial);
+    else
+        col_partial_launch<T, 1>(ctx, rows, dim, n, cblocks, partial);
+    hipLaunchKernelGGL(col_mean_kernel, dim3((dim + 255) / 256), dim3(256), 0, ctx->stream, partial, dim,
+                       cblocks, n, mean);
+    const dim3 rg(static_cast<uint32_t>((n + kThreads - 1) / kThreads));
+    if (row_vectors(rows, static_cast<size_t>(dim) * sizeof(T)))
+        hipLaunchKernelGGL(mean_dist_tiled_kernel<T>, rg, dim3(kThreads), 0, ctx->stream, rows, dim, n,
+                           mean, dist);
+    else
+        hipLaunchKernelGGL(mean_dist_kernel<T>, rg, dim3(kThreads), 0, ctx->stream, rows, dim, n, mean,
+                           dist);
+}
+}  // namespace
+
 int build_medoid(Context* ctx, const void* rows, int elem, uint32_t dim, uint64_t n, uint32_t* out)
 {
     if (int rc = check_elem(ctx, elem)) return rc;
@@ -1565,35 +1732,15 @@ int build_medoid(Context* ctx, const void* rows, int elem, uint32_t dim, uint64_
     double* bd = cv.take<double>(ablocks);
     uint64_t* bi = cv.take<uint64_t>(ablocks);
     uint32_t* res = cv.take<uint32_t>(4);
-    const dim3 cg(static_cast<uint32_t>(cblocks));
-    const dim3 rg(static_cast<uint32_t>((n + 255) / 256));
     switch (elem) {
         case GOFANN_ELEM_U8:
-            hipLaunchKernelGGL(col_partial_kernel<uint8_t>, cg, dim3(kThreads), 0, ctx->stream,
-                               static_cast<const uint8_t*>(rows), dim, n, partial);
+            medoid_dists(ctx, static_cast<const uint8_t*>(rows), dim, n, cblocks, partial, mean, dist);
             break;
         case GOFANN_ELEM_F16:
-            hipLaunchKernelGGL(col_partial_kernel<_Float16>, cg, dim3(kThreads), 0, ctx->stream,
-                               static_cast<const _Float16*>(rows), dim, n, partial);
+            medoid_dists(ctx, static_cast<const _Float16*>(rows), dim, n, cblocks, partial, mean, dist);
             break;
         default:
-            hipLaunchKernelGGL(col_partial_kernel<float>, cg, dim3(kThreads), 0, ctx->stream,
-                               static_cast<const float*>(rows), dim, n, partial);
-    }
-    hipLaunchKernelGGL(col_mean_kernel, dim3((dim + 255) / 256), dim3(256), 0, ctx->stream, partial, dim,
-                       cblocks, n, mean);
-    switch (elem) {
-        case GOFANN_ELEM_U8:
-            hipLaunchKernelGGL(mean_dist_kernel<uint8_t>, rg, dim3(256), 0, ctx->stream,
-                               static_cast<const uint8_t*>(rows), dim, n, mean, dist);
-            break;
-        case GOFANN_ELEM_F16:
-            hipLaunchKernelGGL(mean_dist_kernel<_Float16>, rg, dim3(256), 0, ctx->stream,
-                               static_cast<const _Float16*>(rows), dim, n, mean, dist);
-            break;
-        default:
-            hipLaunchKernelGGL(mean_dist_kernel<float>, rg, dim3(256), 0, ctx->stream,
-                               static_cast<const float*>(rows), dim, n, mean, dist);
+            medoid_dists(ctx, static_cast<const float*>(rows), dim, n, cblocks, partial, mean, dist);
     }
     hipLaunchKernelGGL(argmin_block_kernel, dim3(static_cast<uint32_t>(ablocks)), dim3(kThreads), 0,
                        ctx->stream, dist, n, bd, bi);

@@ -229,3 +229,15 @@ def test_grouping_at_larger_sizes_matches_oracle(hip):
     wp, wg = po.build_cagra_optimize(knn, 32)
     gp_, gg = hip.cagra_optimize(torch.from_numpy(knn.view(np.int32)), 32)
     assert np.array_equal(_u32(gp_), wp) and np.array_equal(_u32(gg), wg)
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("n,dim", [(1, 8), (63, 16), (64, 33), (65, 130), (257, 192), (4095, 64),
+                                   (4097, 31), (8200, 48)])
+def test_medoid_sizes_match_oracle(hip, dtype, n, dim):
+    """Row counts around a wave, a workgroup and a block of column sums; dims
+    whose rows are whole 16-byte vectors, 4-byte words or neither, and
+    several slabs of columns.  All in fp64 in a fixed order: the same row."""
+    say("medoid", dtype.__name__, n, dim)
+    x = _rows(np.random.default_rng(n * 131 + dim), n, dim, dtype)
+    assert hip.medoid(hip.rows(torch.from_numpy(x))) == po.build_medoid(x)
