@@ -366,76 +366,137 @@ __host__ __device__ __forceinline__ double draw_unit(uint64_t seed, uint64_t str
 // k-means++ distance update: best[i] = min(best[i], d(x_i, c)) for the
 // centre picked last (row *pick of the rows), or best[i] = d(x_i, c) when
 // `first`.  One wave per row: lane j sums dims j, j+64, ... (fmaf), then an
-// xor butterfly over offsets 32..1.
+// xor butterfly over offsets 32..1.  One workgroup per chunk of rows (the
+// pick's 1024 chunks), which also adds the chunk's distances in fp64, rows
+// ascending, so that the pick reads 1024 sums instead of every distance.
+constexpr int kKppRows = 32;  // rows of a chunk in one pass of a workgroup
+
 template <class T>
 __global__ __launch_bounds__(kThreads) void kpp_min_kernel(const T* rows, uint32_t dim, uint64_t n,
-                                                           const uint32_t* pick, int first,
-                                                           float* best)
+                                                           uint64_t chunk, const uint32_t* pick,
+                                                           int first, float* best, double* part)
 {
+    constexpr int kWaves = kThreads / kWave;
+    constexpr int kBatch = 4;  // rows of a wave in flight
+    __shared__ float s_best[kKppRows];
     const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
-    const uint64_t r = static_cast<uint64_t>(blockIdx.x) * (kThreads / kWave) + threadIdx.x / kWave;
-    if (r >= n) return;
-    const T* x = rows + r * dim;
+    const int wave = static_cast<int>(threadIdx.x) / kWave;
+    const uint64_t b0 = static_cast<uint64_t>(blockIdx.x) * chunk;
+    const uint64_t b1 = b0 + chunk < n ? b0 + chunk : n;
     const T* c = rows + static_cast<size_t>(*pick) * dim;
-    float s = 0.0f;
-    for (uint32_t d = static_cast<uint32_t>(lane); d < dim; d += kWave) {
-        const float t = to_f(x[d]) - to_f(c[d]);
-        s = fmaf(t, t, s);
-    }
+    double sum = 0.0;
+    for (uint64_t t0 = b0; t0 < b1; t0 += kKppRows) {
+        for (int g = wave * kBatch; g < kKppRows; g += kWaves * kBatch) {
+            if (t0 + g >= b1) break;
+            const T* x[kBatch];
+            float s[kBatch];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, kWave);
-    if (lane == 0) best[r] = first ? s : fminf(best[r], s);
-}
-
-// k-means++ pick: one 1024-thread workgroup.  Thread t sums best over rows
-// [t*chunk, (t+1)*chunk) in fp64 (ascending); thread 0 adds the partial
-// sums in order, sets target = u * total and walks the chunks, then the
-// rows of the chunk, to the first row where the running sum reaches the
-// target (the last row when rounding leaves it short; row floor(u * n) when
-// every distance is zero).  Writes the pick and copies its row to centre j.
-template <class T>
-__global__ __launch_bounds__(1024) void kpp_pick_kernel(const T* rows, uint32_t dim, uint64_t n,
-                                                        const float* best, double u,
-                                                        uint32_t* pick, float* centre)
-{
-    __shared__ double part[1024];
-    __shared__ uint32_t s_pick;
-    const uint32_t t = threadIdx.x;
-    const uint64_t chunk = (n + 1023) / 1024;
-    const uint64_t b0 = static_cast<uint64_t>(t) * chunk;
-    double s = 0.0;
-    for (uint64_t i = b0; i < b0 + chunk && i < n; ++i) s += static_cast<double>(best[i]);
-    part[t] = s;
-    __syncthreads();
-    if (t == 0) {
-        double total = 0.0;
-        for (int i = 0; i < 1024; ++i) total += part[i];
-        uint64_t pk;
-        if (!(total > 0.0)) {
-            pk = static_cast<uint64_t>(u * static_cast<double>(n));
-            if (pk >= n) pk = n - 1;
-        } else {
-            const double target = u * total;
-            double run = 0.0;
-            int c = 0;
-            for (; c < 1023; ++c) {
-                if (run + part[c] >= target) break;
-                run += part[c];
+            for (int i = 0; i < kBatch; ++i) {
+                const uint64_t r = t0 + static_cast<uint64_t>(g + i);
+                x[i] = rows + (r < b1 ? r : b1 - 1) * dim;
+                s[i] = 0.0f;
             }
-            pk = n - 1;
-            const uint64_t e = static_cast<uint64_t>(c + 1) * chunk;
-            for (uint64_t i = static_cast<uint64_t>(c) * chunk; i < e && i < n; ++i) {
-                run += static_cast<double>(best[i]);
-                if (run >= target) {
-                    pk = i;
-                    break;
+#pragma unroll 2
+            for (uint32_t d = static_cast<uint32_t>(lane); d < dim; d += kWave) {
+                const float cv = to_f(c[d]);
+#pragma unroll
+                for (int i = 0; i < kBatch; ++i) {
+                    const float t = to_f(x[i][d]) - cv;
+                    s[i] = fmaf(t, t, s[i]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) {
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) s[i] += __shfl_xor(s[i], off, kWave);
+                const uint64_t r = t0 + static_cast<uint64_t>(g + i);
+                if (lane == 0 && r < b1) {
+                    const float v = first ? s[i] : fminf(best[r], s[i]);
+                    best[r] = v;
+                    s_best[g + i] = v;
                 }
             }
         }
-        s_pick = static_cast<uint32_t>(pk);
-        *pick = s_pick;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int m = static_cast<int>(b1 - t0 < kKppRows ? b1 - t0 : kKppRows);
+            for (int i = 0; i < m; ++i) sum += static_cast<double>(s_best[i]);
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) part[blockIdx.x] = sum;
+}
+
+// k-means++ pick: one 1024-thread workgroup over the chunk sums part[0 ..
+// nchunks).  Thread 0 adds them in order, keeping every running sum (the
+// serial chain that the order asks for, nothing else on it); target =
+// u * the last; the threads then find the first chunk whose running sum
+// reaches it and thread 0 walks that chunk's rows to the first row where
+// the running sum does (the last row when rounding leaves it short; row
+// floor(u * n) when every distance is zero).  Writes the pick and copies
+// its row to centre j.  32,768 x 512 f16 rows, 256 centres: with the chunk sums
+// and a second serial pass in this one workgroup a pick took 45.8 us, now
+// 17.2 (most of it the chain of 1024 adds); the distance update 15.3, now 10.1
+// with four rows of a wave in flight and the chunk sums included.
+template <class T>
+__global__ __launch_bounds__(1024) void kpp_pick_kernel(const T* rows, uint32_t dim, uint64_t n,
+                                                        uint64_t chunk, uint32_t nchunks,
+                                                        const float* best, const double* part,
+                                                        double u, uint32_t* pick, float* centre)
+{
+    __shared__ double s_part[1024];
+    __shared__ double s_run[1025];  // s_run[c]: the sum of chunks 0 .. c - 1
+    __shared__ float s_best[1024];
+    __shared__ uint32_t s_chunk, s_pick;
+    const uint32_t t = threadIdx.x;
+    s_part[t] = t < nchunks ? part[t] : 0.0;
+    if (t == 0) s_chunk = 1023;
+    __syncthreads();
+    if (t == 0) {
+        double run = 0.0;
+        s_run[0] = run;
+#pragma unroll 16
+        for (int i = 0; i < 1024; ++i) {
+            run += s_part[i];
+            s_run[i + 1] = run;
+        }
     }
     __syncthreads();
+    const double total = s_run[1024];
+    const double target = u * total;
+    if (!(total > 0.0)) {
+        if (t == 0) {
+            const uint64_t pk = static_cast<uint64_t>(u * static_cast<double>(n));
+            s_pick = static_cast<uint32_t>(pk < n ? pk : n - 1);
+        }
+    } else {
+        if (t < 1023 && s_run[t + 1] >= target) atomicMin(&s_chunk, t);
+        __syncthreads();
+        const uint64_t b0 = static_cast<uint64_t>(s_chunk) * chunk;
+        const uint64_t b1 = b0 + chunk < n ? b0 + chunk : n;
+        if (t == 0) s_pick = kNone;
+        double run = s_run[s_chunk];
+        for (uint64_t i0 = b0; i0 < b1; i0 += 1024) {
+            if (i0 + t < b1) s_best[t] = best[i0 + t];
+            __syncthreads();
+            if (t == 0) {
+                const int m = static_cast<int>(b1 - i0 < 1024 ? b1 - i0 : 1024);
+                for (int i = 0; i < m; ++i) {
+                    run += static_cast<double>(s_best[i]);
+                    if (run >= target) {
+                        s_pick = static_cast<uint32_t>(i0) + static_cast<uint32_t>(i);
+                        break;
+                    }
+                }
+            }
+            __syncthreads();
+            if (s_pick != kNone) break;  // uniform: every thread reads it after the barrier
+            __syncthreads();
+        }
+        if (t == 0 && s_pick == kNone) s_pick = static_cast<uint32_t>(n - 1);
+    }
+    __syncthreads();
+    if (t == 0) *pick = s_pick;
     const T* x = rows + static_cast<size_t>(s_pick) * dim;
     for (uint32_t d = t; d < dim; d += 1024) centre[d] = to_f(x[d]);
 }
@@ -1339,22 +1400,25 @@ int kmeanspp_t(Context* ctx, const T* rows, uint32_t dim, uint64_t n, uint32_t k
                float* centres)
 {
     unsigned char* buf = static_cast<unsigned char*>(
-        ctx->scratch(Context::kScratchBuild, carve_size({n * 4, 64})));
+        ctx->scratch(Context::kScratchBuild, carve_size({n * 4, 64, 1024 * 8})));
     if (!buf) return ctx->fail(GOFANN_ERR_NOMEM, "k-means++ scratch allocation failed");
     Carve cv{buf, 0};
     float* best = cv.take<float>(n);
     uint32_t* pick = cv.take<uint32_t>(1);
+    double* part = cv.take<double>(1024);
     uint64_t first = static_cast<uint64_t>(draw_unit(seed, 0, 0) * static_cast<double>(n));
     if (first >= n) first = n - 1;
     hipLaunchKernelGGL(first_pick_kernel, dim3(1), dim3(1), 0, ctx->stream,
                        static_cast<uint32_t>(first), pick);
     hipLaunchKernelGGL(copy_row_kernel<T>, dim3(1), dim3(256), 0, ctx->stream, rows, dim, pick, centres);
-    const uint32_t blocks = static_cast<uint32_t>((n + 3) / 4);
+    const uint64_t chunk = (n + 1023) / 1024;
+    const uint32_t nchunks = static_cast<uint32_t>((n + chunk - 1) / chunk);
     for (uint32_t j = 1; j < k; ++j) {
-        hipLaunchKernelGGL(kpp_min_kernel<T>, dim3(blocks), dim3(kThreads), 0, ctx->stream, rows, dim,
-                           n, pick, j == 1 ? 1 : 0, best);
-        hipLaunchKernelGGL(kpp_pick_kernel<T>, dim3(1), dim3(1024), 0, ctx->stream, rows, dim, n, best,
-                           draw_unit(seed, 0, j), pick, centres + static_cast<size_t>(j) * dim);
+        hipLaunchKernelGGL(kpp_min_kernel<T>, dim3(nchunks), dim3(kThreads), 0, ctx->stream, rows, dim,
+                           n, chunk, pick, j == 1 ? 1 : 0, best, part);
+        hipLaunchKernelGGL(kpp_pick_kernel<T>, dim3(1), dim3(1024), 0, ctx->stream, rows, dim, n, chunk,
+                           nchunks, best, part, draw_unit(seed, 0, j), pick,
+                           centres + static_cast<size_t>(j) * dim);
     }
     if (hipGetLastError() != hipSuccess) return ctx->fail_hip("k-means++ launch");
     return GOFANN_OK;

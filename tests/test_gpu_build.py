@@ -241,3 +241,19 @@ def test_medoid_sizes_match_oracle(hip, dtype, n, dim):
     say("medoid", dtype.__name__, n, dim)
     x = _rows(np.random.default_rng(n * 131 + dim), n, dim, dtype)
     assert hip.medoid(hip.rows(torch.from_numpy(x))) == po.build_medoid(x)
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("n,dim,k", [(1, 8, 1), (5, 70, 5), (31, 64, 9), (1023, 33, 6),
+                                     (1025, 130, 6), (40_000, 20, 12)])
+def test_kmeanspp_sizes_match_oracle(hip, dtype, n, dim, k):
+    """Row counts below, at and past the 1024 chunks of the pick (chunks of
+    1, 2 and 40 rows: one and two passes of a workgroup), equal rows (all
+    distances zero once every distinct row is a centre)."""
+    say("k-means++", dtype.__name__, n, dim, k)
+    x = _rows(np.random.default_rng(n * 17 + dim), n, dim, dtype)
+    if n == 31:
+        x[:] = x[:3].repeat(11, axis=0)[:31]
+    want = po.build_kmeanspp(x, k, 7)
+    got = hip.kmeanspp(hip.rows(torch.from_numpy(x)), k, 7)
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
