@@ -780,11 +780,11 @@ __global__ __launch_bounds__(kThreads) void rabitq_encode_kernel(const float* xr
 // a block); the blocks' partial sums are then added in block order.
 constexpr uint32_t kColBlock = 4096;
 
-// Each thread owns kV neighbouring columns of one block of rows and adds them
-// row by row; kColBatch rows are loaded before the first is added, because a
-// chain of one load per add is bound by memory latency (150,000 x 512 f16 in
-// six label groups: 13.9 ms with one column slab a workgroup and one load in
-// flight, 0.55 ms here).  Grid: (row blocks, column slabs of 64 kV).
+// A thread's kV neighbouring columns added row by row over `count` rows;
+// kColBatch rows are loaded before the first is added, because a chain of
+// one load per add is bound by memory latency (150,000 x 512 f16 in six
+// label groups: column sums 13.9 ms with one load in flight and a workgroup
+// per block of rows, 0.55 ms here).
 constexpr int kColBatch = 32;
 
 template <class T, int kV>
@@ -793,21 +793,14 @@ struct alignas(sizeof(T) * kV) Pack {
 };
 
 template <class T, int kV>
-__global__ __launch_bounds__(kWave) void col_partial_kernel(const T* rows, uint32_t dim,
-                                                            uint64_t n, double* partial)
+__device__ __forceinline__ void column_sums(const T* p, uint32_t dim, uint64_t count,
+                                            double (&sum)[kV])
 {
     using P = Pack<T, kV>;
-    const uint64_t b = blockIdx.x;
-    const uint64_t s = b * kColBlock;
-    const uint64_t e = s + kColBlock < n ? s + kColBlock : n;
-    const uint32_t d = (blockIdx.y * kWave + threadIdx.x) * kV;
-    if (d >= dim) return;  // dim is a multiple of kV
-    const T* p = rows + s * dim + d;
-    double sum[kV];
 #pragma unroll
     for (int v = 0; v < kV; ++v) sum[v] = 0.0;
-    uint64_t i = s;
-    for (; i + kColBatch <= e; i += kColBatch) {
+    uint64_t i = 0;
+    for (; i + kColBatch <= count; i += kColBatch) {
         P x[kColBatch];
 #pragma unroll
         for (int t = 0; t < kColBatch; ++t)
@@ -818,11 +811,25 @@ __global__ __launch_bounds__(kWave) void col_partial_kernel(const T* rows, uint3
 #pragma unroll
             for (int v = 0; v < kV; ++v) sum[v] += static_cast<double>(to_f(x[t].v[v]));
     }
-    for (; i < e; ++i, p += dim) {
+    for (; i < count; ++i, p += dim) {
         const P x = *reinterpret_cast<const P*>(p);
 #pragma unroll
         for (int v = 0; v < kV; ++v) sum[v] += static_cast<double>(to_f(x.v[v]));
     }
+}
+
+// Grid: (row blocks, column slabs of 64 kV); dim is a multiple of kV.
+template <class T, int kV>
+__global__ __launch_bounds__(kWave) void col_partial_kernel(const T* rows, uint32_t dim,
+                                                            uint64_t n, double* partial)
+{
+    const uint64_t b = blockIdx.x;
+    const uint64_t s = b * kColBlock;
+    const uint64_t e = s + kColBlock < n ? s + kColBlock : n;
+    const uint32_t d = (blockIdx.y * kWave + threadIdx.x) * kV;
+    if (d >= dim) return;
+    double sum[kV];
+    column_sums<T, kV>(rows + s * dim + d, dim, e - s, sum);
 #pragma unroll
     for (int v = 0; v < kV; ++v) partial[b * dim + d + v] = sum[v];
 }
@@ -1063,6 +1070,93 @@ __global__ __launch_bounds__(kThreads) void bucket_rep_kernel(const T* rows, uin
         __syncthreads();
     }
     if (threadIdx.x == 0) rep[b] = si[0];
+}
+
+// The same representatives in three launches, for rows of whole 16-byte
+// vectors: the means (grid: buckets x column slabs, so that a few buckets of
+// long rows still fill the chip), every row's distance to its bucket's mean
+// (64 rows a wave through tiled_row_chain, whatever their buckets), and the
+// least (distance, row) of each bucket by an unsigned minimum of the pair's
+// bits (distances are not negative; one past FLT_MAX or NaN never wins, as
+// in the kernel above).  50,000 x 512 f16 rows in about 250 buckets: 420 us
+// as one workgroup per bucket, 53 us so.
+template <class T, int kV>
+__global__ __launch_bounds__(kWave) void bucket_mean_kernel(const T* rows, uint32_t dim,
+                                                            const uint32_t* bucket_off,
+                                                            float* means,
+                                                            unsigned long long* keys)
+{
+    const uint32_t b = blockIdx.x;
+    if (blockIdx.y == 0 && threadIdx.x == 0) keys[b] = ~0ull;
+    const uint32_t s = bucket_off[b], e = bucket_off[b + 1];
+    const uint32_t d = (blockIdx.y * kWave + threadIdx.x) * kV;
+    if (s == e || d >= dim) return;
+    double sum[kV];
+    column_sums<T, kV>(rows + static_cast<size_t>(s) * dim + d, dim, e - s, sum);
+#pragma unroll
+    for (int v = 0; v < kV; ++v)
+        means[static_cast<size_t>(b) * dim + d + v] =
+            static_cast<float>(sum[v] / static_cast<double>(e - s));
+}
+
+template <class T>
+__global__ __launch_bounds__(kThreads) void bucket_dist_kernel(const T* rows, uint32_t dim,
+                                                               const uint32_t* bucket_off,
+                                                               uint32_t buckets, uint32_t n,
+                                                               const float* means,
+                                                               unsigned long long* keys)
+{
+    __shared__ uint32_t tiles[(kThreads / kWave) * kRowTileWords];
+    const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+    const int wave = static_cast<int>(threadIdx.x) / kWave;
+    const uint64_t r0 = static_cast<uint64_t>(blockIdx.x) * kThreads + static_cast<uint64_t>(wave) * kWave;
+    if (r0 >= n) return;
+    const uint64_t r = r0 + static_cast<uint64_t>(lane);
+    // the last bucket that starts at or before the row (its rows are never
+    // empty buckets'); rows before the first bucket belong to none
+    uint32_t lo = 0, hi = buckets;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (bucket_off[mid] <= r)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    const bool in = r < n && lo > 0;
+    const uint32_t b = lo > 0 ? lo - 1 : 0;
+    const float* mu = means + static_cast<size_t>(b) * dim;
+    float acc = 0.0f;
+    tiled_row_chain(rows, dim, r0, n, tiles + wave * kRowTileWords, lane,
+                    [&](uint32_t d, const float (&v)[4]) {
+                        const float4 m = *reinterpret_cast<const float4*>(mu + d);
+                        float t = v[0] - m.x;
+                        acc = fmaf(t, t, acc);
+                        t = v[1] - m.y;
+                        acc = fmaf(t, t, acc);
+                        t = v[2] - m.z;
+                        acc = fmaf(t, t, acc);
+                        t = v[3] - m.w;
+                        acc = fmaf(t, t, acc);
+                    });
+    const bool ok = in && acc <= FLT_MAX;
+    uint64_t key = ok ? (static_cast<uint64_t>(__float_as_uint(acc)) << 32) | r : ~0ull;
+    const uint32_t b0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(b)));
+    if (__all(b == b0)) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const uint64_t o = __shfl_xor(static_cast<unsigned long long>(key), off, kWave);
+            key = o < key ? o : key;
+        }
+        if (lane == 0 && key != ~0ull) atomicMin(keys + b0, static_cast<unsigned long long>(key));
+    } else if (ok) {
+        atomicMin(keys + b, static_cast<unsigned long long>(key));
+    }
+}
+
+__global__ void bucket_pick_kernel(const unsigned long long* keys, uint32_t buckets, uint32_t* rep)
+{
+    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b < buckets) rep[b] = static_cast<uint32_t>(keys[b]);  // ~0: kNone
 }
 
 // Link rules of this repo's graph (one wave per row of the bucket-sorted
@@ -1816,6 +1910,34 @@ int build_medoid(Context* ctx, const void* rows, int elem, uint32_t dim, uint64_
     return GOFANN_OK;
 }
 
+namespace {
+template <class T>
+int bucket_reps_t(Context* ctx, const T* rows, uint32_t dim, const uint32_t* bucket_offsets,
+                  uint32_t buckets, uint32_t n, float* means, uint32_t* reps)
+{
+    if (!row_vectors(rows, static_cast<size_t>(dim) * sizeof(T)) ||
+        (reinterpret_cast<uintptr_t>(means) & 15u) != 0) {
+        hipLaunchKernelGGL(bucket_rep_kernel<T>, dim3(buckets), dim3(kThreads), 0, ctx->stream, rows, dim,
+                           bucket_offsets, means, reps);
+    } else {
+        unsigned long long* keys = static_cast<unsigned long long*>(
+            ctx->scratch(Context::kScratchBuild, static_cast<size_t>(buckets) * 8));
+        if (!keys) return ctx->fail(GOFANN_ERR_NOMEM, "bucket representative scratch allocation failed");
+        constexpr int kV = 4 / static_cast<int>(sizeof(T));
+        hipLaunchKernelGGL((bucket_mean_kernel<T, kV>), dim3(buckets, (dim + kWave * kV - 1) / (kWave * kV)),
+                           dim3(kWave), 0, ctx->stream, rows, dim, bucket_offsets, means, keys);
+        if (n > 0)
+            hipLaunchKernelGGL(bucket_dist_kernel<T>, dim3(n / kThreads + (n % kThreads ? 1 : 0)),
+                               dim3(kThreads), 0, ctx->stream, rows, dim, bucket_offsets, buckets, n,
+                               means, keys);
+        hipLaunchKernelGGL(bucket_pick_kernel, dim3((buckets + 255) / 256), dim3(256), 0, ctx->stream,
+                           keys, buckets, reps);
+    }
+    if (hipGetLastError() != hipSuccess) return ctx->fail_hip("bucket representative launch");
+    return GOFANN_OK;
+}
+}  // namespace
+
 int build_bucket_reps(Context* ctx, const void* rows, int elem, uint32_t dim,
                       const uint32_t* bucket_offsets, uint32_t buckets, float* means, uint32_t* reps)
 {
@@ -1823,6 +1945,7 @@ int build_bucket_reps(Context* ctx, const void* rows, int elem, uint32_t dim,
     if (!rows || !bucket_offsets || !means || !reps || dim == 0)
         return ctx->fail(GOFANN_ERR_INVALID, "bucket representatives: arrays missing");
     if (buckets == 0) return GOFANN_OK;
+    uint32_t n = 0;
     {
         std::vector<uint32_t> off(buckets + 1ull);
         if (hipMemcpyAsync(off.data(), bucket_offsets, off.size() * 4, hipMemcpyDeviceToHost,
@@ -1832,22 +1955,19 @@ int build_bucket_reps(Context* ctx, const void* rows, int elem, uint32_t dim,
         for (uint32_t i = 0; i < buckets; ++i)
             if (off[i] > off[i + 1])
                 return ctx->fail(GOFANN_ERR_INVALID, "bucket representatives: offsets decrease");
+        n = off[buckets];
     }
     switch (elem) {
         case GOFANN_ELEM_U8:
-            hipLaunchKernelGGL(bucket_rep_kernel<uint8_t>, dim3(buckets), dim3(kThreads), 0, ctx->stream,
-                               static_cast<const uint8_t*>(rows), dim, bucket_offsets, means, reps);
-            break;
+            return bucket_reps_t(ctx, static_cast<const uint8_t*>(rows), dim, bucket_offsets, buckets, n,
+                                 means, reps);
         case GOFANN_ELEM_F16:
-            hipLaunchKernelGGL(bucket_rep_kernel<_Float16>, dim3(buckets), dim3(kThreads), 0, ctx->stream,
-                               static_cast<const _Float16*>(rows), dim, bucket_offsets, means, reps);
-            break;
+            return bucket_reps_t(ctx, static_cast<const _Float16*>(rows), dim, bucket_offsets, buckets, n,
+                                 means, reps);
         default:
-            hipLaunchKernelGGL(bucket_rep_kernel<float>, dim3(buckets), dim3(kThreads), 0, ctx->stream,
-                               static_cast<const float*>(rows), dim, bucket_offsets, means, reps);
+            return bucket_reps_t(ctx, static_cast<const float*>(rows), dim, bucket_offsets, buckets, n,
+                                 means, reps);
     }
-    if (hipGetLastError() != hipSuccess) return ctx->fail_hip("bucket representative launch");
-    return GOFANN_OK;
 }
 
 int build_links(Context* ctx, const gofann_build_link_inputs* in, const gofann_build_link_params* p,

@@ -257,3 +257,22 @@ def test_kmeanspp_sizes_match_oracle(hip, dtype, n, dim, k):
     want = po.build_kmeanspp(x, k, 7)
     got = hip.kmeanspp(hip.rows(torch.from_numpy(x)), k, 7)
     assert np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("dim", [16, 40, 64, 33, 272])
+def test_bucket_reps_sizes_match_oracle(hip, dtype, dim):
+    """Empty buckets first, between and last, buckets of one row, of about a
+    wave and of several batches of the mean's rows, a wave over several
+    buckets, equal rows (the lowest wins); rows with and without whole
+    16-byte vectors."""
+    say("bucket representatives", dtype.__name__, dim)
+    sizes = [0, 1, 1, 0, 2, 30, 31, 33, 64, 0, 65, 129, 300, 7, 0]
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint32)
+    x = _rows(np.random.default_rng(dim), int(off[-1]), dim, dtype)
+    x[off[8]:off[9]] = x[off[8]]
+    wm, wr = po.build_bucket_reps(x, off)
+    gm, gr = hip.bucket_reps(hip.rows(torch.from_numpy(x)), off)
+    used = np.asarray(sizes) > 0  # an empty bucket's mean is not written
+    assert np.array_equal(_u32(gr), wr)
+    assert np.array_equal(gm.cpu().numpy().view(np.uint32)[used], wm.view(np.uint32)[used])
