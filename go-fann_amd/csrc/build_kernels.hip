@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <cstdint>
 #include <vector>
@@ -54,44 +55,81 @@ __device__ __forceinline__ bool pair_lt(float ad, uint32_t ai, float bd, uint32_
     return ad < bd || (ad == bd && ai < bi);
 }
 
-// Rows [0, n) x dims [d0, d0 + kTileD) of `rows` (row r at rows + r * stride)
-// into lds[dd * kTile + r] as fp32; zero outside the rows and dims.  Thread
-// t takes row t % 64 and eight consecutive dims, so the LDS writes of a
-// wave fall on consecutive banks.
+// A chunk of a tile on its way from memory to LDS: thread t holds eight
+// neighbouring dims, db = d0 + 8 (t % 4), of row t / 4, so four threads read
+// a row's 32 dims back to back.  Requested one chunk ahead and written to LDS
+// after the chunk before it is used up: with the load between two barriers
+// of the same chunk a workgroup waited for memory in every chunk.
+// `vec`: rows of whole 8-element vectors (row_packs), else element by
+// element; zero outside the rows and dims.
 template <class T>
-__device__ __forceinline__ void stage_rows(const T* rows, size_t stride, int n, uint32_t d0,
-                                           uint32_t dim, float* lds, int tid)
+struct alignas(8 * sizeof(T) < 16 ? 8 * sizeof(T) : 16) Pack8 {
+    T v[8];
+};
+
+template <class T>
+__device__ __forceinline__ void chunk_load(const T* rows, size_t stride, int n, uint32_t d0,
+                                           uint32_t dim, bool vec, int tid, Pack8<T>& x)
 {
-    const int r = tid & (kTile - 1);
-    const int g = tid >> 6;  // 0..3
-    const uint32_t db = d0 + static_cast<uint32_t>(g) * 8u;
-    float v[8];
-    if (r < n) {
-        const T* p = rows + static_cast<size_t>(r) * stride;
+    const int r = tid >> 2;
+    const uint32_t db = d0 + static_cast<uint32_t>(tid & 3) * 8u;
+    const T* p = rows + static_cast<size_t>(r < n ? r : 0) * stride;
+    if (vec) {
+        if (r < n && db < dim) {
+            x = *reinterpret_cast<const Pack8<T>*>(p + db);
+        } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = db + i < dim ? to_f(p[db + i]) : 0.0f;
+            for (int i = 0; i < 8; ++i) x.v[i] = static_cast<T>(0);
+        }
     } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = 0.0f;
+        for (int i = 0; i < 8; ++i)
+            x.v[i] = r < n && db + i < dim ? p[db + i] : static_cast<T>(0);
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) lds[(g * 8 + i) * kTile + r] = v[i];
 }
 
-// acc[i][j] += the chunk's terms for rows ty*4+i of sa and tx*4+j of sb
+// ... into lds[dd * kStageStride + r] as fp32.  The stride keeps rows of four
+// 16-byte aligned and puts at most two of a wave's writes on one bank.
+constexpr int kStageStride = kTile + 4;
+
+template <class T>
+__device__ __forceinline__ void chunk_store(const Pack8<T>& x, float* lds, int tid)
+{
+    float* dst = lds + (tid & 3) * 8 * kStageStride + (tid >> 2);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dst[i * kStageStride] = to_f(x.v[i]);
+}
+
+// Whether chunk_load can read `rows` in vectors of eight elements.
+template <class T>
+bool row_packs(const T* rows, uint32_t dim)
+{
+    return dim % 8 == 0 && reinterpret_cast<uintptr_t>(rows) % alignof(Pack8<T>) == 0;
+}
+
+// acc[i][j] += the chunk's terms for rows ty*kI+i of sa and tx*4+j of sb
 // (dims of the chunk ascending; zero-padded dims add exact zeros).
-template <bool kDiff>
+template <bool kDiff, int kI>
 __device__ __forceinline__ void tile_chunk(const float* sa, const float* sb, int ty, int tx,
-                                           float acc[4][4])
+                                           float (&acc)[kI][4])
 {
 #pragma unroll 8
     for (int dd = 0; dd < kTileD; ++dd) {
-        const float4 a = *reinterpret_cast<const float4*>(sa + dd * kTile + ty * 4);
-        const float4 b = *reinterpret_cast<const float4*>(sb + dd * kTile + tx * 4);
-        const float av[4] = {a.x, a.y, a.z, a.w};
+        float av[kI];
+        if constexpr (kI == 4) {
+            const float4 a = *reinterpret_cast<const float4*>(sa + dd * kStageStride + ty * 4);
+            av[0] = a.x;
+            av[1] = a.y;
+            av[2] = a.z;
+            av[3] = a.w;
+        } else {
+#pragma unroll
+            for (int i = 0; i < kI; ++i) av[i] = sa[dd * kStageStride + ty * kI + i];
+        }
+        const float4 b = *reinterpret_cast<const float4*>(sb + dd * kStageStride + tx * 4);
         const float bv[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < kI; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 if (kDiff) {
@@ -123,10 +161,11 @@ __global__ __launch_bounds__(kThreads) void assign_kernel(const T* rows, size_t 
                                                           uint32_t dim, uint64_t n,
                                                           const float* centres,
                                                           const float* cnorm, uint32_t k,
+                                                          bool vec_rows, bool vec_centres,
                                                           uint32_t* out_idx, float* out_score)
 {
-    __shared__ __align__(16) float sa[kTileD * kTile];
-    __shared__ __align__(16) float sb[kTileD * kTile];
+    __shared__ __align__(16) float sa[kTileD * kStageStride];
+    __shared__ __align__(16) float sb[kTileD * kStageStride];
     const int tid = static_cast<int>(threadIdx.x);
     const int ty = tid >> 4, tx = tid & 15;
     const uint64_t r0 = static_cast<uint64_t>(blockIdx.x) * kTile;
@@ -140,6 +179,15 @@ __global__ __launch_bounds__(kThreads) void assign_kernel(const T* rows, size_t 
         best[i] = FLT_MAX;
         bidx[i] = kNone;
     }
+    Pack8<T> xa;
+    Pack8<float> xb;
+    const auto load = [&](uint32_t c0, uint32_t d0) {
+        const int nc = static_cast<int>(k - c0 < kTile ? k - c0 : kTile);
+        chunk_load(qrows, stride, nq, d0, dim, vec_rows, tid, xa);
+        chunk_load(centres + static_cast<size_t>(c0) * dim, static_cast<size_t>(dim), nc, d0, dim,
+                   vec_centres, tid, xb);
+    };
+    load(0, 0);
     for (uint32_t c0 = 0; c0 < k; c0 += kTile) {
         const int nc = static_cast<int>(k - c0 < kTile ? k - c0 : kTile);
         float acc[4][4];
@@ -149,11 +197,14 @@ __global__ __launch_bounds__(kThreads) void assign_kernel(const T* rows, size_t 
             for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
         for (uint32_t d0 = 0; d0 < dim; d0 += kTileD) {
             __syncthreads();
-            stage_rows(qrows, stride, nq, d0, dim, sa, tid);
-            stage_rows(centres + static_cast<size_t>(c0) * dim, static_cast<size_t>(dim), nc, d0,
-                       dim, sb, tid);
+            chunk_store(xa, sa, tid);
+            chunk_store(xb, sb, tid);
             __syncthreads();
-            tile_chunk<false>(sa, sb, ty, tx, acc);
+            if (d0 + kTileD < dim)
+                load(c0, d0 + kTileD);
+            else if (c0 + kTile < k)
+                load(c0 + kTile, 0);
+            tile_chunk<false, 4>(sa, sb, ty, tx, acc);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -198,12 +249,21 @@ __global__ __launch_bounds__(kThreads) void assign_kernel(const T* rows, size_t 
 
 // kNN inside buckets: the rows are sorted by bucket (bucket b holds rows
 // [bucket_off[b], bucket_off[b+1])); query tile t holds rows
-// [tile_row0[t], +64) of bucket tile_bucket[t] and scans the rows of every
+// [tile_row0[t], + kQ) of bucket tile_bucket[t] and scans the rows of every
 // bucket on its probe list (its own bucket when there is no list).  Each
 // query row keeps its k least (distance, row) pairs, itself excluded, in
-// LDS; the lists merge each candidate tile by rank.
-template <class T>
-__global__ __launch_bounds__(kThreads) void knn_kernel(const T* rows, uint32_t dim,
+// LDS; the lists merge each candidate tile by rank.  The tile's distances
+// take the place of the staged chunks, so that LDS holds more workgroups.
+// It is bound by the VALU (a subtraction and an fma per dim of a pair); 50,000
+// x 512 f16 rows in about 250 buckets, k = 16: 1419 us a launch with the
+// chunk loaded between its two barriers, element by element, and the tiles
+// in bucket order; 865 us now (assign_kernel, 32,768 rows x 256 centres: 494,
+// now 264 us).
+constexpr int kKnnStage = 2 * kTileD * kStageStride;  // floats: two chunks, or kQ x 65 distances
+static_assert(kTile * (kTile + 1) <= kKnnStage, "the distances fit the staged chunks");
+
+template <class T, int kQ>
+__global__ __launch_bounds__(kThreads) void knn_kernel(const T* rows, uint32_t dim, bool vec,
                                                        const uint32_t* bucket_off,
                                                        const uint32_t* probe_off,
                                                        const uint32_t* probe,
@@ -211,12 +271,13 @@ __global__ __launch_bounds__(kThreads) void knn_kernel(const T* rows, uint32_t d
                                                        const uint32_t* tile_row0, uint32_t tiles,
                                                        int k, uint32_t* out_ids, float* out_d)
 {
+    constexpr int kI = kQ / 16;                      // query rows per thread
     extern __shared__ __align__(16) unsigned char lds[];
     float* sa = reinterpret_cast<float*>(lds);
-    float* sb = sa + kTileD * kTile;
-    float* sd = sb + kTileD * kTile;                 // [64][65]
-    float* ld_all = sd + kTile * (kTile + 1);        // [64][k]
-    uint32_t* lid_all = reinterpret_cast<uint32_t*>(ld_all + kTile * k);
+    float* sb = sa + kTileD * kStageStride;
+    float* sd = sa;                                  // [kQ][65], after the chunks
+    float* ld_all = sa + kKnnStage;                  // [kQ][k]
+    uint32_t* lid_all = reinterpret_cast<uint32_t*>(ld_all + kQ * k);
     const int tid = static_cast<int>(threadIdx.x);
     const int ty = tid >> 4, tx = tid & 15;
     const int lane = tid & (kWave - 1);
@@ -226,90 +287,115 @@ __global__ __launch_bounds__(kThreads) void knn_kernel(const T* rows, uint32_t d
     const uint32_t b = tile_bucket[t];
     const uint32_t q0 = tile_row0[t];
     const uint32_t qe = bucket_off[b + 1];
-    const int nq = static_cast<int>(qe - q0 < kTile ? qe - q0 : kTile);
-    for (int e = tid; e < kTile * k; e += kThreads) {
+    const int nq = static_cast<int>(qe - q0 < kQ ? qe - q0 : kQ);
+    for (int e = tid; e < kQ * k; e += kThreads) {
         ld_all[e] = FLT_MAX;
         lid_all[e] = kNone;
     }
-    const uint32_t p_begin = probe_off ? probe_off[b] : 0u;
     const uint32_t p_end = probe_off ? probe_off[b + 1] : 1u;
     const T* qrows = rows + static_cast<size_t>(q0) * dim;
-    for (uint32_t p = p_begin; p < p_end; ++p) {
-        const uint32_t pb = probe_off ? probe[p] : b;
-        const uint32_t c_begin = bucket_off[pb], c_end = bucket_off[pb + 1];
-        for (uint32_t c0 = c_begin; c0 < c_end; c0 += kTile) {
-            const int nc = static_cast<int>(c_end - c0 < kTile ? c_end - c0 : kTile);
-            float acc[4][4];
+    // candidate tiles in order: rows [c0, min(c0 + 64, c_end)) of probe p
+    uint32_t p = probe_off ? probe_off[b] : 0u, c0 = 0, c_end = 0;
+    const auto open = [&]() {  // the first rows at or after probe p; false: none are left
+        for (; p < p_end; ++p) {
+            const uint32_t pb = probe_off ? probe[p] : b;
+            c0 = bucket_off[pb];
+            c_end = bucket_off[pb + 1];
+            if (c0 < c_end) return true;
+        }
+        return false;
+    };
+    Pack8<T> xa, xb;
+    const auto load = [&](uint32_t d0) {
+        chunk_load(qrows, static_cast<size_t>(dim), nq, d0, dim, vec, tid, xa);
+        chunk_load(rows + static_cast<size_t>(c0) * dim, static_cast<size_t>(dim),
+                   static_cast<int>(c_end - c0 < kTile ? c_end - c0 : kTile), d0, dim, vec, tid, xb);
+    };
+    bool more = open();
+    if (more) load(0);
+    while (more) {
+        const uint32_t tile0 = c0;
+        const int nc = static_cast<int>(c_end - c0 < kTile ? c_end - c0 : kTile);
+        float acc[kI][4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < kI; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-            for (uint32_t d0 = 0; d0 < dim; d0 += kTileD) {
-                __syncthreads();
-                stage_rows(qrows, static_cast<size_t>(dim), nq, d0, dim, sa, tid);
-                stage_rows(rows + static_cast<size_t>(c0) * dim, static_cast<size_t>(dim), nc, d0,
-                           dim, sb, tid);
-                __syncthreads();
-                tile_chunk<true>(sa, sb, ty, tx, acc);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) sd[(ty * 4 + i) * (kTile + 1) + tx * 4 + j] = acc[i][j];
+            for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
+        for (uint32_t d0 = 0; d0 < dim; d0 += kTileD) {
             __syncthreads();
-            // wave w merges the tile into the lists of rows w*16 .. w*16+15
-            for (int ii = 0; ii < kTile / 4; ++ii) {
-                const int qi = wave * (kTile / 4) + ii;
-                if (qi >= nq) break;
-                const uint32_t self = q0 + static_cast<uint32_t>(qi);
-                float* ld = ld_all + qi * k;
-                uint32_t* lid = lid_all + qi * k;
-                const uint32_t cid = c0 + static_cast<uint32_t>(lane);
-                const float v = sd[qi * (kTile + 1) + lane];
-                const bool valid = lane < nc && cid != self;
-                const bool in = valid && pair_lt(v, cid, ld[k - 1], lid[k - 1]);
-                const uint64_t sm = __ballot(in);
-                if (!sm) continue;
-                int c_self = 0;
-                if (in) {
-                    int lo = 0, hi = k;
-                    while (lo < hi) {
-                        const int mid = (lo + hi) >> 1;
-                        if (pair_lt(ld[mid], lid[mid], v, cid))
-                            lo = mid + 1;
-                        else
-                            hi = mid;
-                    }
-                    c_self = lo;
+            if (kQ == kTile || tid < kQ * 4) chunk_store(xa, sa, tid);
+            chunk_store(xb, sb, tid);
+            __syncthreads();
+            if (d0 + kTileD < dim) {
+                load(d0 + kTileD);
+            } else {
+                c0 += kTile;
+                if (c0 >= c_end) {
+                    ++p;
+                    more = open();
                 }
-                const int e0 = lane, e1 = lane + kWave;
-                const float d0v = e0 < k ? ld[e0] : FLT_MAX;
-                const uint32_t i0 = e0 < k ? lid[e0] : kNone;
-                const float d1v = e1 < k ? ld[e1] : FLT_MAX;
-                const uint32_t i1 = e1 < k ? lid[e1] : kNone;
-                int c0n = 0, c1n = 0;
-                for (uint64_t m = sm; m; m &= m - 1) {
-                    const int src = __builtin_ctzll(m);
-                    const float sv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
-                    const uint32_t si = static_cast<uint32_t>(
-                        __builtin_amdgcn_readlane(static_cast<int>(cid), src));
-                    c0n += pair_lt(sv, si, d0v, i0) ? 1 : 0;
-                    c1n += pair_lt(sv, si, d1v, i1) ? 1 : 0;
-                    c_self += pair_lt(sv, si, v, cid) ? 1 : 0;
+                if (more) load(0);
+            }
+            tile_chunk<true, kI>(sa, sb, ty, tx, acc);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kI; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sd[(ty * kI + i) * (kTile + 1) + tx * 4 + j] = acc[i][j];
+        __syncthreads();
+        // wave w merges the tile into the lists of its kQ / 4 rows
+        for (int ii = 0; ii < kQ / 4; ++ii) {
+            const int qi = wave * (kQ / 4) + ii;
+            if (qi >= nq) break;
+            const uint32_t self = q0 + static_cast<uint32_t>(qi);
+            float* ld = ld_all + qi * k;
+            uint32_t* lid = lid_all + qi * k;
+            const uint32_t cid = tile0 + static_cast<uint32_t>(lane);
+            const float v = sd[qi * (kTile + 1) + lane];
+            const bool valid = lane < nc && cid != self;
+            const bool in = valid && pair_lt(v, cid, ld[k - 1], lid[k - 1]);
+            const uint64_t sm = __ballot(in);
+            if (!sm) continue;
+            int c_self = 0;
+            if (in) {
+                int lo = 0, hi = k;
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (pair_lt(ld[mid], lid[mid], v, cid))
+                        lo = mid + 1;
+                    else
+                        hi = mid;
                 }
-                // all reads of the old list precede these writes (one wave)
-                if (e0 < k && e0 + c0n < k) {
-                    ld[e0 + c0n] = d0v;
-                    lid[e0 + c0n] = i0;
-                }
-                if (e1 < k && e1 + c1n < k) {
-                    ld[e1 + c1n] = d1v;
-                    lid[e1 + c1n] = i1;
-                }
-                if (in && c_self < k) {
-                    ld[c_self] = v;
-                    lid[c_self] = cid;
-                }
+                c_self = lo;
+            }
+            const int e0 = lane, e1 = lane + kWave;
+            const float d0v = e0 < k ? ld[e0] : FLT_MAX;
+            const uint32_t i0 = e0 < k ? lid[e0] : kNone;
+            const float d1v = e1 < k ? ld[e1] : FLT_MAX;
+            const uint32_t i1 = e1 < k ? lid[e1] : kNone;
+            int c0n = 0, c1n = 0;
+            for (uint64_t m = sm; m; m &= m - 1) {
+                const int src = __builtin_ctzll(m);
+                const float sv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
+                const uint32_t si = static_cast<uint32_t>(
+                    __builtin_amdgcn_readlane(static_cast<int>(cid), src));
+                c0n += pair_lt(sv, si, d0v, i0) ? 1 : 0;
+                c1n += pair_lt(sv, si, d1v, i1) ? 1 : 0;
+                c_self += pair_lt(sv, si, v, cid) ? 1 : 0;
+            }
+            // all reads of the old list precede these writes (one wave)
+            if (e0 < k && e0 + c0n < k) {
+                ld[e0 + c0n] = d0v;
+                lid[e0 + c0n] = i0;
+            }
+            if (e1 < k && e1 + c1n < k) {
+                ld[e1 + c1n] = d1v;
+                lid[e1 + c1n] = i1;
+            }
+            if (in && c_self < k) {
+                ld[c_self] = v;
+                lid[c_self] = cid;
             }
         }
     }
@@ -318,29 +404,6 @@ __global__ __launch_bounds__(kThreads) void knn_kernel(const T* rows, uint32_t d
         const size_t o = static_cast<size_t>(q0) * k + static_cast<size_t>(e);
         out_ids[o] = lid_all[e];
         if (out_d) out_d[o] = ld_all[e];
-    }
-}
-
-__global__ void knn_tile_count_kernel(const uint32_t* bucket_off, uint32_t buckets,
-                                      uint32_t* counts)
-{
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= buckets) return;
-    const uint32_t n = bucket_off[b + 1] - bucket_off[b];
-    counts[b] = (n + kTile - 1) / kTile;
-}
-
-__global__ void knn_tile_fill_kernel(const uint32_t* bucket_off, uint32_t buckets,
-                                     const uint32_t* tile_off, uint32_t* tile_bucket,
-                                     uint32_t* tile_row0)
-{
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= buckets) return;
-    const uint32_t s = bucket_off[b], e = bucket_off[b + 1];
-    uint32_t t = tile_off[b];
-    for (uint32_t r = s; r < e; r += kTile, ++t) {
-        tile_bucket[t] = b;
-        tile_row0[t] = r;
     }
 }
 
@@ -1432,7 +1495,8 @@ int assign_t(Context* ctx, const void* rows, uint32_t dim, uint64_t n, const flo
     const uint64_t blocks = (n + kTile - 1) / kTile;
     hipLaunchKernelGGL(assign_kernel<T>, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0,
                        ctx->stream, static_cast<const T*>(rows), static_cast<size_t>(dim), dim, n,
-                       centres, cnorm, k, out_idx, out_score);
+                       centres, cnorm, k, row_packs(static_cast<const T*>(rows), dim),
+                       row_packs(centres, dim), out_idx, out_score);
     if (hipGetLastError() != hipSuccess) return ctx->fail_hip("assign launch");
     return GOFANN_OK;
 }
@@ -1538,7 +1602,8 @@ int kmeans_t(Context* ctx, const T* rows, uint32_t dim, uint64_t n, uint32_t k, 
                            k, dim, cnorm);
         hipLaunchKernelGGL(assign_kernel<T>, dim3(static_cast<uint32_t>((n + kTile - 1) / kTile)),
                            dim3(kThreads), 0, ctx->stream, rows, static_cast<size_t>(dim), dim, n,
-                           centres, cnorm, k, idx, static_cast<float*>(nullptr));
+                           centres, cnorm, k, row_packs(rows, dim), row_packs(centres, dim), idx,
+                           static_cast<float*>(nullptr));
         // the rows of each centre in ascending order
         if (hipMemsetAsync(counts, 0, (static_cast<size_t>(k) + 1) * 4, ctx->stream) != hipSuccess)
             return ctx->fail_hip("k-means counts clear");
@@ -1562,72 +1627,84 @@ int knn_t(Context* ctx, const T* rows, uint32_t dim, const gofann_build_buckets*
     const uint32_t nb = b->buckets;
     // The bucket and probe arrays index the rows: check them on the host
     // (they are small) before any kernel reads through them.
-    {
-        std::vector<uint32_t> off(nb + 1ull);
-        if (hipMemcpyAsync(off.data(), b->bucket_offsets, off.size() * 4, hipMemcpyDeviceToHost,
+    std::vector<uint32_t> off(nb + 1ull), po, pb;
+    if (hipMemcpyAsync(off.data(), b->bucket_offsets, off.size() * 4, hipMemcpyDeviceToHost,
+                       ctx->stream) != hipSuccess ||
+        hipStreamSynchronize(ctx->stream) != hipSuccess)
+        return ctx->fail_hip("kNN bucket offsets copy");
+    for (uint32_t i = 0; i < nb; ++i)
+        if (off[i] > off[i + 1]) return ctx->fail(GOFANN_ERR_INVALID, "kNN: bucket offsets decrease");
+    if (off[nb] != b->rows) return ctx->fail(GOFANN_ERR_INVALID, "kNN: bucket offsets do not end at rows");
+    if (b->probe_offsets) {
+        po.resize(nb + 1ull);
+        if (hipMemcpyAsync(po.data(), b->probe_offsets, po.size() * 4, hipMemcpyDeviceToHost,
                            ctx->stream) != hipSuccess ||
             hipStreamSynchronize(ctx->stream) != hipSuccess)
-            return ctx->fail_hip("kNN bucket offsets copy");
+            return ctx->fail_hip("kNN probe offsets copy");
         for (uint32_t i = 0; i < nb; ++i)
-            if (off[i] > off[i + 1]) return ctx->fail(GOFANN_ERR_INVALID, "kNN: bucket offsets decrease");
-        if (off[nb] != b->rows) return ctx->fail(GOFANN_ERR_INVALID, "kNN: bucket offsets do not end at rows");
-        if (b->probe_offsets) {
-            std::vector<uint32_t> po(nb + 1ull);
-            if (hipMemcpyAsync(po.data(), b->probe_offsets, po.size() * 4, hipMemcpyDeviceToHost,
-                               ctx->stream) != hipSuccess ||
-                hipStreamSynchronize(ctx->stream) != hipSuccess)
-                return ctx->fail_hip("kNN probe offsets copy");
-            for (uint32_t i = 0; i < nb; ++i)
-                if (po[i] > po[i + 1]) return ctx->fail(GOFANN_ERR_INVALID, "kNN: probe offsets decrease");
-            std::vector<uint32_t> pb(po[nb]);
-            if (!pb.empty() &&
-                (hipMemcpyAsync(pb.data(), b->probe_buckets, pb.size() * 4, hipMemcpyDeviceToHost,
-                                ctx->stream) != hipSuccess ||
-                 hipStreamSynchronize(ctx->stream) != hipSuccess))
-                return ctx->fail_hip("kNN probe buckets copy");
-            for (uint32_t i = 0; i < nb; ++i)
-                for (uint32_t q = po[i]; q < po[i + 1]; ++q) {
-                    if (pb[q] >= nb) return ctx->fail(GOFANN_ERR_INVALID, "kNN: probe bucket out of range");
-                    for (uint32_t q2 = po[i]; q2 < q; ++q2)
-                        if (pb[q2] == pb[q]) return ctx->fail(GOFANN_ERR_INVALID, "kNN: a probe list repeats a bucket");
-                }
-        }
+            if (po[i] > po[i + 1]) return ctx->fail(GOFANN_ERR_INVALID, "kNN: probe offsets decrease");
+        pb.resize(po[nb]);
+        if (!pb.empty() &&
+            (hipMemcpyAsync(pb.data(), b->probe_buckets, pb.size() * 4, hipMemcpyDeviceToHost,
+                            ctx->stream) != hipSuccess ||
+             hipStreamSynchronize(ctx->stream) != hipSuccess))
+            return ctx->fail_hip("kNN probe buckets copy");
+        for (uint32_t i = 0; i < nb; ++i)
+            for (uint32_t q = po[i]; q < po[i + 1]; ++q) {
+                if (pb[q] >= nb) return ctx->fail(GOFANN_ERR_INVALID, "kNN: probe bucket out of range");
+                for (uint32_t q2 = po[i]; q2 < q; ++q2)
+                    if (pb[q2] == pb[q]) return ctx->fail(GOFANN_ERR_INVALID, "kNN: a probe list repeats a bucket");
+            }
     }
-    // query tiles per bucket: counts, exclusive sum, fill
-    // (tiles <= rows / 64 + buckets)
-    const size_t max_tiles = static_cast<size_t>(b->rows) / kTile + nb + 1;
-    unsigned char* buf = static_cast<unsigned char*>(ctx->scratch(
-        Context::kScratchBuild,
-        carve_size({(nb + 1ull) * 4, (nb + 1ull) * 4, max_tiles * 4, max_tiles * 4})));
-    if (!buf) return ctx->fail(GOFANN_ERR_NOMEM, "kNN scratch allocation failed");
-    Carve cv{buf, 0};
-    uint32_t* counts = cv.take<uint32_t>(nb + 1ull);
-    uint32_t* tile_off = cv.take<uint32_t>(nb + 1ull);
-    uint32_t* tile_bucket = cv.take<uint32_t>(max_tiles);
-    uint32_t* tile_row0 = cv.take<uint32_t>(max_tiles);
-    hipLaunchKernelGGL(knn_tile_count_kernel, dim3((nb + 255) / 256), dim3(256), 0, ctx->stream,
-                       b->bucket_offsets, nb, counts);
-    hipLaunchKernelGGL(exclusive_scan_kernel, dim3(1), dim3(1024), 0, ctx->stream, counts,
-                       static_cast<uint64_t>(nb), tile_off);
-    uint32_t tiles = 0;
-    if (hipMemcpyAsync(&tiles, tile_off + nb, 4, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
-        hipStreamSynchronize(ctx->stream) != hipSuccess)
-        return ctx->fail_hip("kNN tile count");
-    if (tiles > max_tiles) return ctx->fail(GOFANN_ERR_INVALID, "kNN: bucket offsets exceed the rows");
+    // Buckets by falling number of candidates, so that the tiles that scan
+    // longest start first and the last workgroups are short.
+    std::vector<uint64_t> cand(nb);
+    std::vector<uint32_t> by(nb);
+    uint64_t whole = 0;
+    for (uint32_t i = 0; i < nb; ++i) {
+        by[i] = i;
+        cand[i] = off[i + 1] - off[i];
+        if (b->probe_offsets) {
+            cand[i] = 0;
+            for (uint32_t q = po[i]; q < po[i + 1]; ++q) cand[i] += off[pb[q] + 1] - off[pb[q]];
+        }
+        whole += (off[i + 1] - off[i] + kTile - 1) / kTile;
+    }
+    std::stable_sort(by.begin(), by.end(), [&](uint32_t x, uint32_t y) { return cand[x] > cand[y]; });
+    // Query tiles of 64 rows, or of 16 where 64 would leave most of the chip
+    // without a tile (256 centres of 512 dims, k = 4, is 4 tiles of 64:
+    // 459 us, as 16 of 16 rows 113 us).
+    const int kq = whole < static_cast<uint64_t>(ctx->compute_units) ? 16 : kTile;
+    std::vector<uint32_t> list;  // bucket of every tile, then first row of every tile
+    for (uint32_t i : by)
+        for (uint64_t r = off[i]; r < off[i + 1]; r += kq) list.push_back(i);
+    const uint32_t tiles = static_cast<uint32_t>(list.size());
     if (tiles == 0) return GOFANN_OK;
-    hipLaunchKernelGGL(knn_tile_fill_kernel, dim3((nb + 255) / 256), dim3(256), 0, ctx->stream,
-                       b->bucket_offsets, nb, tile_off, tile_bucket, tile_row0);
-    const size_t lds = (2 * kTileD * kTile + kTile * (kTile + 1)) * 4 + static_cast<size_t>(kTile) * k * 8;
+    for (uint32_t i : by)
+        for (uint64_t r = off[i]; r < off[i + 1]; r += kq) list.push_back(static_cast<uint32_t>(r));
+    uint32_t* dev = static_cast<uint32_t*>(ctx->scratch(Context::kScratchBuild, list.size() * 4));
+    if (!dev) return ctx->fail(GOFANN_ERR_NOMEM, "kNN scratch allocation failed");
+    if (hipMemcpyAsync(dev, list.data(), list.size() * 4, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
+        return ctx->fail_hip("kNN tile list copy");
+    const size_t lds = (kKnnStage + static_cast<size_t>(kq) * k * 2) * 4;
     if (lds > static_cast<size_t>(ctx->lds_per_block))
         return ctx->fail(GOFANN_ERR_UNSUPPORTED, "kNN list exceeds the workgroup LDS");
-    const void* kern = reinterpret_cast<const void*>(knn_kernel<T>);
-    if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) !=
-        hipSuccess)
-        return ctx->fail_hip("hipFuncSetAttribute kNN");
-    hipLaunchKernelGGL(knn_kernel<T>, dim3(tiles), dim3(kThreads), lds, ctx->stream, rows, dim,
-                       b->bucket_offsets, b->probe_offsets, b->probe_buckets, tile_bucket, tile_row0,
-                       tiles, static_cast<int>(k), out_ids, out_d);
-    if (hipGetLastError() != hipSuccess) return ctx->fail_hip("kNN launch");
+    const auto launch = [&](auto kern) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                static_cast<int>(lds)) != hipSuccess)
+            return ctx->fail_hip("hipFuncSetAttribute kNN");
+        hipLaunchKernelGGL(kern, dim3(tiles), dim3(kThreads), lds, ctx->stream, rows, dim,
+                           row_packs(rows, dim), b->bucket_offsets, b->probe_offsets,
+                           b->probe_buckets, dev, dev + tiles, tiles, static_cast<int>(k), out_ids,
+                           out_d);
+        if (hipGetLastError() != hipSuccess) return ctx->fail_hip("kNN launch");
+        return GOFANN_OK;
+    };
+    if (int rc = kq == kTile ? launch(knn_kernel<T, kTile>) : launch(knn_kernel<T, 16>)) {
+        (void)hipStreamSynchronize(ctx->stream);  // the tile list is still being copied
+        return rc;
+    }
     // the scratch is reused by the next call: finish here
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) return ctx->fail_hip("kNN synchronize");
     return GOFANN_OK;

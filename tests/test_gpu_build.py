@@ -276,3 +276,19 @@ def test_bucket_reps_sizes_match_oracle(hip, dtype, dim):
     used = np.asarray(sizes) > 0  # an empty bucket's mean is not written
     assert np.array_equal(_u32(gr), wr)
     assert np.array_equal(gm.cpu().numpy().view(np.uint32)[used], wm.view(np.uint32)[used])
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("dim", [8, 31, 36, 200])
+def test_knn_many_tiles_match_oracle(hip, dtype, dim):
+    """More 64-row tiles than the chip has compute units (64-row query
+    tiles; the other kNN tests take the 16-row ones), buckets of very
+    different sizes, rows with and without whole 8-element vectors."""
+    say("knn tiles", dtype.__name__, dim)
+    rng = np.random.default_rng(dim * 3 + 1)
+    sizes = np.concatenate([rng.integers(1, 30, size=270), [300, 129, 0, 64, 65]])
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint32)
+    x = _rows(rng, int(off[-1]), dim, dtype)
+    want, _ = po.build_knn(x, off, 16)
+    got = hip.knn(hip.rows(torch.from_numpy(x)), off, 16)
+    assert np.array_equal(_u32(got), want)
