@@ -61,6 +61,19 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t x)
 }
 
 
+// The same for the maximum.
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x)
+{
+    x = max(x, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0xB1, 0xF, 0xF, false)));
+    x = max(x, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x4E, 0xF, 0xF, false)));
+    x = max(x, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x141, 0xF, 0xF, false)));
+    x = max(x, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x140, 0xF, 0xF, false)));
+    const uint32_t a = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 0));
+    const uint32_t b = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 16));
+    const uint32_t c = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 32));
+    const uint32_t d = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 48));
+    return max(max(a, b), max(c, d));
+}
 
 constexpr uint32_t kHashCapacity = 4096;  // backend_pq.cu:194
 constexpr int kMaxDegree = 64;            // include/config1B.h:29 FIXED_DEGREE
@@ -77,6 +90,12 @@ struct alignas(16) Entry {  // one 16-byte LDS access per entry
     uint32_t second;
     float base;
     uint32_t sample;
+};
+
+// A heap entry reduced to what its order needs: the key and which entry it is.
+struct alignas(8) HeapPair {
+    float first;
+    uint32_t second;
 };
 
 struct ResultEntry {  // KernelPair<dist_t, uint32_t>
@@ -417,6 +436,22 @@ __device__ __forceinline__ Entry shfl_entry(const Entry& e, int src)
     return r;
 }
 
+__device__ __forceinline__ HeapPair shfl_entry(const HeapPair& e, int src)
+{
+    HeapPair r;
+    r.first = __int_as_float(__shfl(__float_as_int(e.first), src, kWave));
+    r.second = static_cast<uint32_t>(__shfl(static_cast<int>(e.second), src, kWave));
+    return r;
+}
+
+__device__ __forceinline__ HeapPair readlane_entry(const HeapPair& e, int src)
+{
+    HeapPair r;
+    r.first = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e.first), src));
+    r.second = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(e.second), src));
+    return r;
+}
+
 __device__ __forceinline__ Entry readlane_entry(const Entry& e, int src)
 {
     Entry r;
@@ -458,7 +493,35 @@ __device__ __forceinline__ Entry select_entry(bool c, const Entry& a, const Entr
     return r;
 }
 
-__device__ __forceinline__ void wave_smmh_insert(Entry* h, int& size, const Entry& e, int lane)
+__device__ __forceinline__ HeapPair select_entry(bool c, const HeapPair& a, const HeapPair& b)
+{
+    HeapPair r;
+    r.first = c ? a.first : b.first;
+    r.second = c ? a.second : b.second;
+    return r;
+}
+
+// Lane i's entry becomes lane i + 1's (within rows of 16 lanes).
+__device__ __forceinline__ Entry row_next(const Entry& e)
+{
+    Entry r;
+    r.first = dpp_row_f<kDppRowShl1>(e.first, e.first);
+    r.second = static_cast<uint32_t>(dpp_row<kDppRowShl1>(static_cast<int>(e.second), static_cast<int>(e.second)));
+    r.base = dpp_row_f<kDppRowShl1>(e.base, e.base);
+    r.sample = static_cast<uint32_t>(dpp_row<kDppRowShl1>(static_cast<int>(e.sample), static_cast<int>(e.sample)));
+    return r;
+}
+__device__ __forceinline__ HeapPair row_next(const HeapPair& e)
+{
+    HeapPair r;
+    r.first = dpp_row_f<kDppRowShl1>(e.first, e.first);
+    r.second = static_cast<uint32_t>(dpp_row<kDppRowShl1>(static_cast<int>(e.second), static_cast<int>(e.second)));
+    return r;
+}
+
+// E: Entry or HeapPair.
+template <class E>
+__device__ __forceinline__ void wave_smmh_insert(E* h, int& size, const E& e, int lane)
 {
     const int y0 = __builtin_amdgcn_readfirstlane(size);
     size = y0 + 1;
@@ -468,9 +531,9 @@ __device__ __forceinline__ void wave_smmh_insert(Entry* h, int& size, const Entr
     const bool act = lane >= 1 && lane <= depth;
     // lanes past the chain read slots 1 and 2 (inside the frontier) and stay out
     const int a1 = act ? 2 * (((pair + 1) >> lane) - 1) + 1 : 1;
-    const Entry al = h[a1];
-    const Entry ar = h[a1 + 1];
-    const Entry sib = h[y0 - 1];
+    const E al = h[a1];
+    const E ar = h[a1 + 1];
+    const E sib = h[y0 - 1];
     // bottom sibling step: the pair's left entry moves right (lane 63 writes it)
     const bool moved =
         !(y0 & 1) && e.first < __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(sib.first)));
@@ -483,7 +546,7 @@ __device__ __forceinline__ void wave_smmh_insert(Entry* h, int& size, const Entr
         else if (__int_as_float(__builtin_amdgcn_readlane(__float_as_int(ar.first), 1)) < e.first)
             side = 1;
     }
-    const Entry v = select_entry(side == 1, ar, al);
+    const E v = select_entry(side == 1, ar, al);
     const float sg = side == 1 ? -1.0f : 1.0f;  // climb: v > e on the left side, v < e on the right
     const uint64_t mask = ballot(side >= 0 && act && sg * v.first > sg * e.first);
     const int t = __builtin_ctzll(~(mask >> 1));  // levels climbed (0 when it stays)
@@ -491,7 +554,7 @@ __device__ __forceinline__ void wave_smmh_insert(Entry* h, int& size, const Entr
     // lane 0: the new entry; lanes 1..t: the chain moves down one level
     const int lv = lane == 0 ? t : lane - 1;
     int dst = lv == 0 ? y : 2 * (((pair + 1) >> lv) - 1) + 1 + sd;
-    Entry w = select_entry(lane == 0, e, v);
+    E w = select_entry(lane == 0, e, v);
     bool wr = lane == 0 || (act && lane <= t);
     if (lane == kWave - 1) {
         dst = y0;
@@ -502,11 +565,12 @@ __device__ __forceinline__ void wave_smmh_insert(Entry* h, int& size, const Entr
 }
 
 // Returns the new maximum (slot 2's `first`); the heap keeps >= 3 slots.
-__device__ __forceinline__ float wave_smmh_pop_max(Entry* h, int& size, int lane)
+template <class E>
+__device__ __forceinline__ float wave_smmh_pop_max(E* h, int& size, int lane)
 {
     const int n = __builtin_amdgcn_readfirstlane(size) - 1;
     size = n;
-    const Entry v = h[n];  // the last entry replaces the maximum
+    const E v = h[n];  // the last entry replaces the maximum
     // bit q: pair q's larger child is its right one (ties: the left)
     uint64_t pick0, pick1 = 0;
     {
@@ -531,8 +595,8 @@ __device__ __forceinline__ float wave_smmh_pop_max(Entry* h, int& size, int lane
     // lane k <= depth: path slot k; lanes past the path read slot 2
     const int k = lane <= depth ? lane : 0;
     const int slot = 2 * (((p + 1) >> (depth - k)) - 1) + 2;
-    const Entry R = h[slot];
-    const Entry L = h[slot - 1];
+    const E R = h[slot];
+    const E L = h[slot - 1];
     float x = L.first;
     const float ninf = -__builtin_inff();
     x = fmaxf(x, dpp_row_f<kDppRowShr1>(ninf, x));
@@ -542,19 +606,15 @@ __device__ __forceinline__ float wave_smmh_pop_max(Entry* h, int& size, int lane
     const float vf = fmaxf(v.first, x);                        // after level `lane`
     const float prev = dpp_row_f<kDppRowShr1>(v.first, vf);    // entering level `lane`
     const uint64_t swapped = ballot(lane <= depth && L.first > prev);
-    Entry rnext;  // path slot lane + 1
-    rnext.first = dpp_row_f<kDppRowShl1>(R.first, R.first);
-    rnext.second = static_cast<uint32_t>(dpp_row<kDppRowShl1>(static_cast<int>(R.second), static_cast<int>(R.second)));
-    rnext.base = dpp_row_f<kDppRowShl1>(R.base, R.base);
-    rnext.sample = static_cast<uint32_t>(dpp_row<kDppRowShl1>(static_cast<int>(R.sample), static_cast<int>(R.sample)));
+    const E rnext = row_next(R);  // path slot lane + 1
     const int stop = __builtin_ctzll(~ballot(lane < depth && rnext.first > vf));
     // entering level k: the last left entry swapped in above k, else v
     const uint64_t above = swapped & ((1ull << lane) - 1ull);
-    const Entry lsrc = shfl_entry(L, above ? 63 - __builtin_clzll(above) : 0);
+    const E lsrc = shfl_entry(L, above ? 63 - __builtin_clzll(above) : 0);
     // where it stops: the left entry swapped in there or above, else v
     const uint64_t upto = swapped & ((2ull << stop) - 1ull);
-    const Entry lfin = readlane_entry(L, upto ? 63 - __builtin_clzll(upto) : 0);
-    const Entry fin = select_entry(upto != 0, lfin, v);
+    const E lfin = readlane_entry(L, upto ? 63 - __builtin_clzll(upto) : 0);
+    const E fin = select_entry(upto != 0, lfin, v);
     if (lane <= stop) {
         h[slot] = select_entry(lane == stop, fin, rnext);
         if ((swapped >> lane) & 1ull) h[slot - 1] = select_entry(above != 0, lsrc, v);

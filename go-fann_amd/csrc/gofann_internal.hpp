@@ -22,7 +22,8 @@ struct Context {
         kScratchMisc = 2,
         kScratchRange = 3,  // per-segment range-scan shortlists before the merge
         kScratchBuild = 4,  // index construction (k-means, kNN, graph optimisation)
-        kScratchCount = 5
+        kScratchLog = 5,    // admission logs of the set frontier
+        kScratchCount = 6
     };
 
     int device = 0;

@@ -318,3 +318,89 @@ def test_exact_search_rejects_bad_params(gpu_ctx, eworld):
                                              _lib.ptr(q), dg.view(), None, _lib.PredicateView(),
                                              dr.routes_view(), prm, None, None, None)
         assert rc in (_lib.ERR_INVALID, _lib.ERR_UNSUPPORTED)
+
+
+# ---- the set frontier (set_frontier.hpp) -------------------------------
+@pytest.mark.parametrize("shift", [4, 6, 7])
+@pytest.mark.parametrize("Q", [2, 7, 48, 111, 112, 113, 240, 241, 496, 497])
+def test_exact_search_equal_distances(gpu_ctx, eworld, shift, Q):
+    """Beams around every register count of the set frontier (112, 240 and
+    496 are the last of two, four and eight; 497 takes the heap) over rows
+    of 16, 4 and 2 distinct values a dim: many equal distances, so that the
+    order of the heap decides who is next and who leaves."""
+    wl, li, rs = eworld
+    say("exact search, equal distances", shift, "Q", Q)
+    rows = (wl.base.numpy()[:, :12] >> shift, wl.queries.numpy()[:, :12] >> shift)
+    rows = tuple(np.ascontiguousarray(r) for r in rows)
+
+    class Small:
+        dim, n = 12, wl.n
+        base, queries = wl.base, wl.queries
+    _run(gpu_ctx, Small, li, rs, None, lambda dr, dg: _lib.PredicateView(), Q, 10, 2,
+         _lib.PLACE_AUTO, False, rows=rows)
+
+
+def _run_both(ctx, li, rs, base, q, Q, mode):
+    """gofann_exact_search (set frontier) and gofann_exact_search_noalloc
+    (heap frontier) on the same inputs."""
+    dg, dr = gs.DeviceGraph.upload(li), gs.DeviceRoutes.upload(rs)
+    b, qd = torch.from_numpy(base).cuda(), torch.from_numpy(q).cuda()
+    ls = gs.u32(li.label_size)
+    out = []
+    for fn in (ctx.lib.gofann_exact_search, ctx.lib.gofann_exact_search_noalloc):
+        n = rs.count
+        ids = torch.empty(n * 10, dtype=torch.int32, device="cuda")
+        dists = torch.empty(n * 10, device="cuda")
+        st = torch.zeros(n * 8, dtype=torch.int32, device="cuda")
+        prm = _lib.ExactParams(Q, 1, mode, 0, 10, _lib.PLACE_AUTO)
+        ctx.check(fn(ctx.handle, _lib.ptr(b), ELEM[base.dtype], base.shape[1], base.shape[0],
+                     _lib.ptr(qd), dg.view(), _lib.ptr(ls), _lib.PredicateView(),
+                     dr.routes_view(), prm, _lib.ptr(ids), _lib.ptr(dists), _lib.ptr(st)))
+        torch.cuda.synchronize()
+        out.append([ids.cpu().numpy(), dists.cpu().numpy().view(np.uint32), st.cpu().numpy()])
+    return out
+
+
+@pytest.mark.parametrize("Q", [8, 96, 200, 448])
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+@pytest.mark.parametrize("kind", ["nan", "inf", "zero", "huge"])
+def test_exact_search_unordered_distances(gpu_ctx, eworld, dtype, Q, kind):
+    """NaN, infinite, all-zero and overflowing distances: the set frontier
+    gives what the heap frontier gives."""
+    wl, li, rs = eworld
+    say("exact search", kind, dtype, "Q", Q)
+    rng = np.random.default_rng(Q)
+    base = (rng.standard_normal((wl.n, 24))).astype(np.float32)
+    q = (rng.standard_normal((wl.queries.shape[0], 24))).astype(np.float32)
+    hit = rng.random(wl.n) < 0.1
+    if kind == "nan":
+        base[hit, 3] = np.nan
+        base[rng.random(wl.n) < 0.02, 5] = -np.nan
+    elif kind == "inf":
+        base[hit, 3] = np.inf
+        base[rng.random(wl.n) < 0.1, 5] = -np.inf
+        q[::3, 3] = np.inf
+    elif kind == "zero":
+        base[:] = 0
+        q[::2] = 0
+    else:
+        base[hit] *= 1e20 if dtype == "f32" else 1e4
+    dt = np.float32 if dtype == "f32" else np.float16
+    with np.errstate(over="ignore"):
+        a, b = _run_both(gpu_ctx, li, rs, base.astype(dt), q.astype(dt), Q, 2)
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
+
+
+def test_exact_search_log_ring_wraps(gpu_ctx, eworld):
+    """Routes without early stop admit more entries than the log ring of a
+    small beam holds (1024), so that the ring brings the heap up to date."""
+    wl, li, rs = eworld
+    say("exact search, log ring")
+    rng = np.random.default_rng(3)
+    base = rng.standard_normal((wl.n, 32)).astype(np.float32)
+    q = rng.standard_normal((wl.queries.shape[0], 32)).astype(np.float32)
+    for Q in (112, 496):
+        a, b = _run_both(gpu_ctx, li, rs, base, q, Q, 1)
+        for x, y in zip(a, b):
+            assert np.array_equal(x, y)
