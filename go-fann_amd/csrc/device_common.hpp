@@ -93,7 +93,7 @@ struct alignas(16) Entry {  // one 16-byte LDS access per entry
 };
 
 // A heap entry reduced to what its order needs: the key and which entry it is.
-struct alignas(8) HeapPair {
+struct HeapPair {
     float first;
     uint32_t second;
 };
@@ -145,6 +145,21 @@ __device__ __forceinline__ int opaque_lane(int lane)
     return lane;
 }
 
+// A kernel's arguments, T at `offset` bytes of the kernarg segment, behind an
+// empty asm statement.  A route loop that takes them from here at the top of
+// every step reads each field again by a scalar load where it is used;
+// otherwise the compiler loads all of them once, has no scalar registers for
+// them over the whole route, and keeps them in lanes of vector registers
+// (a v_readlane per word and use).
+template <class T>
+__device__ __forceinline__ const T& step_args(uint32_t offset = 0)
+{
+    typedef const __attribute__((address_space(4))) char* Ptr;
+    Ptr p = (Ptr)__builtin_amdgcn_kernarg_segment_ptr() + offset;
+    asm volatile("" : "+s"(p));
+    return *(const T*)p;
+}
+
 // ---------------------------------------------------------------------------
 // Visited set: native_visited_hash.cuh:10-60.  Observable semantics: an exact
 // set of label-local rows that stops accepting values once it holds 4096 of
@@ -175,7 +190,9 @@ constexpr uint32_t kSpillSlots = 1024;
 constexpr uint32_t kSpillLimit = kSpillSlots * 3 / 4;
 
 // Linear-probing table over `cap` slots (a power of two dividing 4096).
-template <bool kShared>
+// kWindow (global slabs): test reads aligned windows of four slots, so that a
+// probe past a few neighbours is one trip to memory.
+template <bool kShared, bool kWindow = false>
 struct ProbeTable {
     uint32_t* slots;
     uint32_t cap;
@@ -202,13 +219,36 @@ struct ProbeTable {
     __device__ bool test(uint32_t value) const
     {
         uint32_t slot = hash_code(value) & (cap - 1);
-        for (uint32_t probes = 0; probes < cap; ++probes) {
-            const uint32_t v = load(slot);
-            if (v == UINT32_MAX) return false;
-            if (v == value) return true;
-            slot = (slot + 1) & (cap - 1);
+        if constexpr (!kWindow) {
+            for (uint32_t probes = 0; probes < cap; ++probes) {
+                const uint32_t v = load(slot);
+                if (v == UINT32_MAX) return false;
+                if (v == value) return true;
+                slot = (slot + 1) & (cap - 1);
+            }
+            return false;
+        } else {
+            uint32_t from = slot & 3u;
+            slot &= ~3u;
+            for (uint32_t probes = 0; probes <= cap; probes += 4) {
+                const uint64_t* w = reinterpret_cast<const uint64_t*>(slots + slot);
+                const uint64_t lo = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint64_t hi = __hip_atomic_load(w + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t v[4] = {static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32),
+                                       static_cast<uint32_t>(hi), static_cast<uint32_t>(hi >> 32)};
+                // the first slot of the window, from the value's own on, that
+                // decides
+                int found = -1;
+#pragma unroll
+                for (int t = 3; t >= 0; --t)
+                    if (static_cast<uint32_t>(t) >= from && (v[t] == UINT32_MAX || v[t] == value))
+                        found = v[t] == value ? 1 : 0;
+                if (found >= 0) return found != 0;
+                from = 0;
+                slot = (slot + 4) & (cap - 1);
+            }
+            return false;
         }
-        return false;
     }
     // Serial insert: 1 when stored, 0 when present or the table is full.
     __device__ int add(uint32_t value) const
@@ -250,7 +290,7 @@ struct ProbeTable {
 template <int kMode>
 struct VisitedSet {
     ProbeTable<true> shared;    // LDS table (kVisitedLds, kVisitedSpill)
-    ProbeTable<false> global;   // global slab of 4096 slots
+    ProbeTable<false, kMode == kVisitedGlobal> global;  // global slab of 4096 slots
     uint32_t count;             // values held (wave-uniform)
     bool spilled;               // kVisitedSpill: moved to the global slab
 
@@ -519,9 +559,30 @@ __device__ __forceinline__ HeapPair row_next(const HeapPair& e)
     return r;
 }
 
-// E: Entry or HeapPair.
-template <class E>
-__device__ __forceinline__ void wave_smmh_insert(E* h, int& size, const E& e, int lane)
+// A heap of HeapPairs as two arrays (6 bytes a slot).
+struct SplitHeap {
+    float* first;
+    uint16_t* second;
+};
+
+// Slot access of the two heap forms (Entry array, SplitHeap).
+__device__ __forceinline__ Entry heap_get(const Entry* h, int i) { return h[i]; }
+__device__ __forceinline__ float heap_key(const Entry* h, int i) { return h[i].first; }
+__device__ __forceinline__ void heap_set(Entry* h, int i, const Entry& e) { h[i] = e; }
+__device__ __forceinline__ HeapPair heap_get(const SplitHeap& h, int i)
+{
+    return HeapPair{h.first[i], h.second[i]};
+}
+__device__ __forceinline__ float heap_key(const SplitHeap& h, int i) { return h.first[i]; }
+__device__ __forceinline__ void heap_set(const SplitHeap& h, int i, const HeapPair& e)
+{
+    h.first[i] = e.first;
+    h.second[i] = static_cast<uint16_t>(e.second);
+}
+
+// H: Entry* with E = Entry, or SplitHeap with E = HeapPair.
+template <class H, class E>
+__device__ __forceinline__ void wave_smmh_insert(H h, int& size, const E& e, int lane)
 {
     const int y0 = __builtin_amdgcn_readfirstlane(size);
     size = y0 + 1;
@@ -531,9 +592,9 @@ __device__ __forceinline__ void wave_smmh_insert(E* h, int& size, const E& e, in
     const bool act = lane >= 1 && lane <= depth;
     // lanes past the chain read slots 1 and 2 (inside the frontier) and stay out
     const int a1 = act ? 2 * (((pair + 1) >> lane) - 1) + 1 : 1;
-    const E al = h[a1];
-    const E ar = h[a1 + 1];
-    const E sib = h[y0 - 1];
+    const E al = heap_get(h, a1);
+    const E ar = heap_get(h, a1 + 1);
+    const E sib = heap_get(h, y0 - 1);
     // bottom sibling step: the pair's left entry moves right (lane 63 writes it)
     const bool moved =
         !(y0 & 1) && e.first < __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(sib.first)));
@@ -561,27 +622,27 @@ __device__ __forceinline__ void wave_smmh_insert(E* h, int& size, const E& e, in
         w = sib;
         wr = moved;
     }
-    if (wr) h[dst] = w;
+    if (wr) heap_set(h, dst, w);
 }
 
 // Returns the new maximum (slot 2's `first`); the heap keeps >= 3 slots.
-template <class E>
-__device__ __forceinline__ float wave_smmh_pop_max(E* h, int& size, int lane)
+template <class H>
+__device__ __forceinline__ float wave_smmh_pop_max(H h, int& size, int lane)
 {
     const int n = __builtin_amdgcn_readfirstlane(size) - 1;
     size = n;
-    const E v = h[n];  // the last entry replaces the maximum
+    const auto v = heap_get(h, n);  // the last entry replaces the maximum
     // bit q: pair q's larger child is its right one (ties: the left)
     uint64_t pick0, pick1 = 0;
     {
         const int cl = 4 * lane + 4;
         const int cr = cl + 2;
-        const float fl = h[min(cl, n - 1)].first;
-        const float fr = h[min(cr, n - 1)].first;
+        const float fl = heap_key(h, min(cl, n - 1));
+        const float fr = heap_key(h, min(cr, n - 1));
         pick0 = ballot(cr < n && fr > fl);
         if (n > 260) {
-            const float gl = h[min(cl + 256, n - 1)].first;
-            const float gr = h[min(cr + 256, n - 1)].first;
+            const float gl = heap_key(h, min(cl + 256, n - 1));
+            const float gr = heap_key(h, min(cr + 256, n - 1));
             pick1 = ballot(cr + 256 < n && gr > gl);
         }
     }
@@ -595,8 +656,8 @@ __device__ __forceinline__ float wave_smmh_pop_max(E* h, int& size, int lane)
     // lane k <= depth: path slot k; lanes past the path read slot 2
     const int k = lane <= depth ? lane : 0;
     const int slot = 2 * (((p + 1) >> (depth - k)) - 1) + 2;
-    const E R = h[slot];
-    const E L = h[slot - 1];
+    const auto R = heap_get(h, slot);
+    const auto L = heap_get(h, slot - 1);
     float x = L.first;
     const float ninf = -__builtin_inff();
     x = fmaxf(x, dpp_row_f<kDppRowShr1>(ninf, x));
@@ -606,18 +667,18 @@ __device__ __forceinline__ float wave_smmh_pop_max(E* h, int& size, int lane)
     const float vf = fmaxf(v.first, x);                        // after level `lane`
     const float prev = dpp_row_f<kDppRowShr1>(v.first, vf);    // entering level `lane`
     const uint64_t swapped = ballot(lane <= depth && L.first > prev);
-    const E rnext = row_next(R);  // path slot lane + 1
+    const auto rnext = row_next(R);  // path slot lane + 1
     const int stop = __builtin_ctzll(~ballot(lane < depth && rnext.first > vf));
     // entering level k: the last left entry swapped in above k, else v
     const uint64_t above = swapped & ((1ull << lane) - 1ull);
-    const E lsrc = shfl_entry(L, above ? 63 - __builtin_clzll(above) : 0);
+    const auto lsrc = shfl_entry(L, above ? 63 - __builtin_clzll(above) : 0);
     // where it stops: the left entry swapped in there or above, else v
     const uint64_t upto = swapped & ((2ull << stop) - 1ull);
-    const E lfin = readlane_entry(L, upto ? 63 - __builtin_clzll(upto) : 0);
-    const E fin = select_entry(upto != 0, lfin, v);
+    const auto lfin = readlane_entry(L, upto ? 63 - __builtin_clzll(upto) : 0);
+    const auto fin = select_entry(upto != 0, lfin, v);
     if (lane <= stop) {
-        h[slot] = select_entry(lane == stop, fin, rnext);
-        if ((swapped >> lane) & 1ull) h[slot - 1] = select_entry(above != 0, lsrc, v);
+        heap_set(h, slot, select_entry(lane == stop, fin, rnext));
+        if ((swapped >> lane) & 1ull) heap_set(h, slot - 1, select_entry(above != 0, lsrc, v));
     }
     return stop == 0 ? fin.first : __int_as_float(__builtin_amdgcn_readlane(__float_as_int(R.first), 1));
 }
@@ -1120,7 +1181,8 @@ __device__ __forceinline__ bool pickup(Entry* f, int size, Entry& out, int lane,
     const uint32_t mn = wave_min_u32(bk);
     if (mn == UINT32_MAX) return false;
     const int best = static_cast<int>(wave_min_u32(bk == mn ? bi : UINT32_MAX));
-    out = f[best];
+    // uniform, so in scalar registers
+    out = readlane_entry(f[best], 0);
     __syncthreads();
     if (lane == 0) f[best].second |= kPoolUsed;
     __syncthreads();

@@ -204,17 +204,26 @@ static int exact_search_impl(Context* ctx, const void* base, int base_elem, uint
     // float rows over kQuadMaxRowBytes take the long-row kernel
     const int fchunks = static_cast<size_t>(dim) * elem_bytes(base_elem) > kQuadMaxRowBytes ? -1 : 0;
     const uint32_t q = static_cast<uint32_t>(p->queue_limit);
-    if (const int regs = fixed_slab == nullptr ? set_registers(ctx, p->queue_limit, r->count, &a.log) : 0) {
+    // The set frontier serves float rows, whose distances are seldom equal
+    // (4,900 f16 routes, dim 512: 9.9 ms, 10.5 with the heap), and u8
+    // launches of at most 16 routes: a u8 route without equal
+    // keys that matter runs in two thirds of the heap's time (248 against 369
+    // us), but one that has them replays its admissions on the heap, so the
+    // slowest of many is slower than with the heap (280 routes 1.16 against
+    // 1.04 ms), and a full chip's average is no better.
+    const bool set_pays = base_elem != GOFANN_ELEM_U8 || r->count <= 16;
+    if (const int regs = fixed_slab == nullptr && set_pays
+                             ? set_registers(ctx, p->queue_limit, r->count, &a.log) : 0) {
         a.log_mask = set_log_entries(p->queue_limit) - 1u;
         a.off_heap = align16u(a.off_frontier + set_capacity(p->queue_limit, regs) * 8u);
-        layout(a.off_heap - a.off_frontier + (q + 2u) * static_cast<uint32_t>(sizeof(HeapPair)));
+        layout(a.off_heap - a.off_frontier + split_heap_bytes(p->queue_limit));
         int rc;
         switch (base_elem) {
         case GOFANN_ELEM_F32: rc = launch_set<GOFANN_ELEM_F32>(sh, fchunks, regs); break;
         case GOFANN_ELEM_F16: rc = launch_set<GOFANN_ELEM_F16>(sh, fchunks, regs); break;
         default: rc = launch_set<GOFANN_ELEM_U8>(sh, 0, regs); break;
         }
-        // (the set takes 112 bytes of LDS more than the heap)
+        // (below 64 slots the set takes more LDS than the heap)
         if (rc != GOFANN_ERR_UNSUPPORTED) return rc;
     }
     const int chunks = (GOFANN_EXACT_FIXED_ROWS && (dim == 128 || dim == 192 || dim == 256))

@@ -27,17 +27,18 @@ constexpr int kExactMaxTopk = 10;  // defaults::max_topk
 #endif
 
 // Minimum waves per SIMD the u8 kernels are compiled for (register budget).
-// 6 holds them to 80 VGPRs, 24 routes per CU, without spills (the lane id is
-// opaque per step).  At C2, Q = 80: 46.1 ms, against 49.0 at 5 waves and
-// 54.1 at 7 (the visited table leaves LDS).  The f32 / f16 kernels (eight
-// partial sums and two 16-byte loads per lane) take 5: at 6 they spill.
+// 6 holds them to 80 VGPRs, 24 routes per CU, without spills (the lane id and
+// the arguments are taken anew per step).  At C2, Q = 80: 46.1 ms, against 49.0
+// at 5 waves and 54.1 at 7 (the visited table leaves LDS).  The f32 / f16 kernels
+// (eight partial sums and two 16-byte loads per lane) take 5: at 6 they spill.
 #ifndef GOFANN_EXACT_MIN_WAVES
 #define GOFANN_EXACT_MIN_WAVES 6
 #endif
 
 // 16-byte row chunks loaded per memory round trip in the any-dim row loop.
-// At 6 waves, C2, Q = 80: three take 49.0 ms, four 46.1, six 48.9, the whole
-// row (twelve) 47.5.
+// With one chunk's query words in registers at a time four fit the 80 VGPRs
+// without spills; 57,000 routes of 192 bytes, Q = 72: three take 13.6 ms, four
+// 12.5, six (four registers spilled) 12.5.
 #ifndef GOFANN_EXACT_ROW_UNROLL
 #define GOFANN_EXACT_ROW_UNROLL 4
 #endif
@@ -89,9 +90,7 @@ __device__ __forceinline__ uint32_t l2_u8_row(const uint8_t* row, const uint32_t
     if ((dim & 15u) == 0) {
         const uint4* r4 = reinterpret_cast<const uint4*>(row);
         const uint4* q4 = reinterpret_cast<const uint4*>(q);
-#pragma unroll kU
-        for (uint32_t i = 0; i < dim / 16; ++i) {
-            const uint4 b = r4[i];
+        const auto add = [&](const uint4& b, uint32_t i) {
             const uint4 w = q4[i];
             nb = __builtin_amdgcn_udot4(b.x, b.x, nb, false);
             nb = __builtin_amdgcn_udot4(b.y, b.y, nb, false);
@@ -101,7 +100,21 @@ __device__ __forceinline__ uint32_t l2_u8_row(const uint8_t* row, const uint32_t
             dot = __builtin_amdgcn_udot4(b.y, w.y, dot, false);
             dot = __builtin_amdgcn_udot4(b.z, w.z, dot, false);
             dot = __builtin_amdgcn_udot4(b.w, w.w, dot, false);
+        };
+        const uint32_t n = dim / 16;
+        uint32_t i = 0;
+        for (; i + kU <= n; i += kU) {
+            uint4 b[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) b[u] = r4[i + u];
+            // one chunk's query words in registers at a time
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                add(b[u], i + u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
+        for (; i < n; ++i) add(r4[i], i);
         return nb + qnorm - 2u * dot;
     }
     if ((dim & 3u) == 0) {
@@ -318,7 +331,7 @@ __device__ __forceinline__ float wave_float_dists(const uint8_t* base, uint32_t 
 // kR: 0, the frontier is the heap in LDS; else a set of kR registers a lane
 // (set_frontier.hpp).
 template <int kVisited, int kC, int kElem, int kR>
-__device__ __forceinline__ void exact_route(const ExactArgs& a, unsigned char* lds)
+__device__ __forceinline__ void exact_route(const ExactArgs& args, unsigned char* lds)
 {
     constexpr int kRowUnroll = GOFANN_EXACT_ROW_UNROLL;
     constexpr bool kSet = kR > 0;
@@ -327,6 +340,7 @@ __device__ __forceinline__ void exact_route(const ExactArgs& a, unsigned char* l
     __shared__ float s_dist[kMaxDegree];
     __shared__ uint64_t s_adm;
 
+    const ExactArgs& a = args;
     const int lane = static_cast<int>(threadIdx.x);
     const uint32_t slot = xcd_slot(blockIdx.x, gridDim.x);
     if (slot >= a.routes.count) return;
@@ -337,7 +351,7 @@ __device__ __forceinline__ void exact_route(const ExactArgs& a, unsigned char* l
 
     uint32_t* qw = reinterpret_cast<uint32_t*>(lds);
     Entry* frontier = reinterpret_cast<Entry*>(lds + a.off_frontier);
-    SetFrontier<kSet ? kR : 1, false, kElem != GOFANN_ELEM_U8> set;
+    SetFrontier<kSet ? kR : 1, kElem != GOFANN_ELEM_U8> set;
     VisitedSet<kVisited> visited;
 
     const uint32_t group = a.routes.route_group[route];
@@ -408,10 +422,10 @@ __device__ __forceinline__ void exact_route(const ExactArgs& a, unsigned char* l
             }
             const Entry kp = {d0, seed, d0, s0};
             if constexpr (kSet) {
-                set.init(reinterpret_cast<uint2*>(lds + a.off_frontier), nullptr,
-                         reinterpret_cast<HeapPair*>(lds + a.off_heap),
+                set.init(reinterpret_cast<uint2*>(lds + a.off_frontier),
+                         split_heap(lds + a.off_heap, Q),
                          a.log + static_cast<size_t>(slot) * (a.log_mask + 1), a.log_mask, Q);
-                set.seed(d0, seed, d0, s0, lane);
+                set.seed(d0, seed, s0, lane);
                 now = kp;
             } else {
                 if (lane == 0) smmh_insert(frontier, heap_size, kp);
@@ -439,8 +453,11 @@ __device__ __forceinline__ void exact_route(const ExactArgs& a, unsigned char* l
     const int wave_lane = lane;
     while (!done) {
         // per step: lane-derived values are not held across steps (no spills
-        // at 6 waves; with the lane hoisted out of the loop, 10 VGPRs spilled)
+        // at 6 waves; with the lane hoisted out of the loop, 10 VGPRs spilled),
         const int lane = opaque_lane(wave_lane);
+        // nor are the arguments (105-128 scalar registers spilled into vector
+        // lanes, 8-18 now)
+        const ExactArgs& a = step_args<ExactArgs>();
         if (a.params.max_steps != 0 && steps >= static_cast<uint32_t>(a.params.max_steps)) break;
 
         // One memory round for the neighbours (visited tests, sample ids) and
@@ -507,7 +524,7 @@ __device__ __forceinline__ void exact_route(const ExactArgs& a, unsigned char* l
         // during the step), then admit the rest in adjacency order.
         uint64_t adm = 0;  // admitted lanes
         if constexpr (kSet) {
-            adm = set.admit(keep, dist, adj, dist, samp, lane);
+            adm = set.admit(keep, dist, adj, samp, lane);
         } else {
             const bool full = heap_size > 2 && heap_size >= Q + 1;
             const float thr = full ? frontier[2].first : 0.0f;
@@ -582,8 +599,7 @@ __device__ __forceinline__ void exact_route(const ExactArgs& a, unsigned char* l
         // Pickup and early stop (:1985-2030).
         bool found;
         if constexpr (kSet) {
-            float unused;
-            found = set.pickup(next, lane, false, unused);
+            found = set.pickup(next, lane);
         } else {
             found = pickup(frontier, heap_size, next, lane);
         }
@@ -640,9 +656,8 @@ __global__ __launch_bounds__(64, (kElem == GOFANN_ELEM_U8 ? GOFANN_EXACT_MIN_WAV
     exact_route<kVisited, kC, kElem, 0>(a, lds);
 }
 
-// (eight registers a lane of u8 beams: 6 waves per SIMD spill 50 VGPRs)
 template <int kVisited, int kC, int kElem, int kR>
-__global__ __launch_bounds__(64, (kElem != GOFANN_ELEM_U8 ? GOFANN_EXACT_FLOAT_MIN_WAVES : kR == 8 ? 5 : GOFANN_EXACT_MIN_WAVES)) void exact_set_kernel(ExactArgs a)
+__global__ __launch_bounds__(64, 4) void exact_set_kernel(ExactArgs a)
 {
     extern __shared__ __align__(16) unsigned char lds[];
     exact_route<kVisited, kC, kElem, kR>(a, lds);
@@ -679,7 +694,7 @@ int exact_resident(Context* ctx, uint32_t lds)
 // Visited-set placement, then the launch.  Auto: the full LDS table, else the
 // spilling one, where every route of the launch is resident with it; else the
 // most resident routes per CU, the global slab only where it holds a quarter
-// more of them (u8, Q = 72, 57,000 routes: 28 a CU with the slab take 12.15 ms,
+// more of them (u8, Q = 72, 57,000 routes: 28 a CU with the slab took 12.15 ms,
 // 24 with the spilling table 12.11).
 // fixed_slab: visited slabs for a placement outside LDS, holding at most
 // fixed_routes routes (the no-alloc entry point); nullptr: context scratch.

@@ -22,10 +22,9 @@
 //     rest of them leave too, which is what mostly happens; if one of them is
 //     about to be picked, the heap says which are left.
 // Of 380 admissions of a u8 route at Q = 72 (integer distances, so keys meet
-// often) the heap saw 84, of 1,100 of an f16 route at Q = 416 it saw 15.
-// Exact routes, heap and set: one u8 route 492 and 302 us, 280 routes 1.51 and
-// 1.34 ms, 57,000 routes 12.7 and 12.1 ms (the base rows' traffic bounds those),
-// 4,900 f16 routes 10.2 and 9.8 ms.
+// often) the heap saw 84, of 1,100 of an f16 route at Q = 416 it saw 15.  One u8
+// route takes 248 us, with the heap 369; which launches take it, and why not
+// all, is said where they are chosen (exact_route.hip).
 // A NaN key has no place in such an order: from the first one on (eager) every
 // admission goes through the heap as well.
 #pragma once
@@ -41,6 +40,17 @@
 namespace gofann {
 
 constexpr uint32_t kSetSlack = 16;  // positions past Q for entries whose leaving is open
+
+// LDS bytes of a SplitHeap for a beam of q (Q + 2 slots).
+__host__ __device__ inline uint32_t split_heap_bytes(int q)
+{
+    return (static_cast<uint32_t>(q) + 2u) * 6u;
+}
+__device__ __forceinline__ SplitHeap split_heap(unsigned char* lds, int q)
+{
+    float* f = reinterpret_cast<float*>(lds);
+    return SplitHeap{f, reinterpret_cast<uint16_t*>(f + q + 2)};
+}
 
 // Positions of a beam of q in r registers a lane.
 __host__ __device__ inline uint32_t set_capacity(int q, int r)
@@ -63,18 +73,16 @@ __device__ __forceinline__ void static_for(F&& f)
     static_for_(f, std::make_integer_sequence<int, N>{});
 }
 
-// R registers a lane.  kBase: entries carry an unbiased score of their own
-// (else it is the key).  kNan: keys may be NaN.
-template <int R, bool kBase, bool kNan>
+// R registers a lane.  kNan: keys may be NaN.
+template <int R, bool kNan>
 struct SetFrontier {
     static_assert(R >= 1 && R <= 8, "the heap operations hold 512 slots");
     static constexpr uint32_t kDone = UINT32_MAX;
     using Keys = uint32_t __attribute__((ext_vector_type(R)));
     Keys key;          // order key of a position; 0: free
-    Keys pick;         // the same while the entry is unused; kDone: free or used
+    uint32_t unused;   // bit i: register i holds an unused entry
     uint2* entry;      // LDS [cap]: row, sample
-    float* base;       // LDS [cap] (kBase)
-    HeapPair* heap;    // LDS [Q + 2]: key and position
+    SplitHeap heap;    // LDS [Q + 2]: key and position
     uint64_t* log;     // this route's ring of admitted (position, key bits)
     uint32_t log_mask;
     uint32_t cap;
@@ -88,15 +96,12 @@ struct SetFrontier {
     int top_gone;               // how many of those have left the frontier
     bool eager;
 
-    __device__ void init(uint2* entry_, float* base_, HeapPair* heap_, uint64_t* log_,
-                         uint32_t log_mask_, int q)
+    __device__ void init(uint2* entry_, const SplitHeap& heap_, uint64_t* log_, uint32_t log_mask_,
+                         int q)
     {
-        static_for<R>([&](auto i) {
-            key[int{i}] = 0u;
-            pick[int{i}] = kDone;
-        });
+        static_for<R>([&](auto i) { key[int{i}] = 0u; });
+        unused = 0u;
         entry = entry_;
-        base = base_;
         heap = heap_;
         log = log_;
         log_mask = log_mask_;
@@ -110,15 +115,20 @@ struct SetFrontier {
         eager = false;
     }
 
-    __device__ __forceinline__ void put(int pos, uint32_t k, uint32_t p, int lane)
+    // Position pos takes key k (0: it is free).
+    __device__ __forceinline__ void put(int pos, uint32_t k, bool is_unused, int lane)
     {
         const bool me = lane == (pos & (kWave - 1));
         static_for<R>([&](auto i) {
-            if ((pos >> 6) == i) {
-                key[int{i}] = me ? k : key[int{i}];
-                pick[int{i}] = me ? p : pick[int{i}];
-            }
+            if ((pos >> 6) == i) key[int{i}] = me ? k : key[int{i}];
         });
+        const uint32_t bit = me ? 1u << (pos >> 6) : 0u;
+        unused = is_unused ? unused | bit : unused & ~bit;
+    }
+    // The key of register i where its entry is unused.
+    __device__ __forceinline__ uint32_t pick(int i, uint32_t k) const
+    {
+        return (unused >> i) & 1u ? k : kDone;
     }
     __device__ __forceinline__ int free_pos(int lane) const
     {
@@ -175,10 +185,10 @@ struct SetFrontier {
                 const int l = __builtin_ctzll(m);
                 bool in = false;
                 for (int s = lane + 1; s < heap_size; s += kWave)
-                    in |= heap[s].second == static_cast<uint32_t>(64 * i + l);
+                    in |= heap.second[s] == static_cast<uint32_t>(64 * i + l);
                 if (!ballot(in) && lane == l) {
                     key[int{i}] = 0u;
-                    pick[int{i}] = kDone;
+                    unused &= ~(1u << i);
                 }
             }
         });
@@ -187,41 +197,40 @@ struct SetFrontier {
     }
 
     // The first entry (held by every lane), already marked used.
-    __device__ __forceinline__ void seed(float first, uint32_t row, float b, uint32_t sample, int lane)
+    __device__ __forceinline__ void seed(float first, uint32_t row, uint32_t sample, int lane)
     {
         const uint32_t k = order_key(first);
         if constexpr (kNan) {
             if (first != first) {
                 eager = true;
-                if (lane == 0) heap[1] = HeapPair{first, 0u};
+                if (lane == 0) heap_set(heap, 1, HeapPair{first, 0u});
                 heap_size = 2;
             }
         }
-        place(0, 0, max(k, 1u), kDone, first, row, b, sample, lane);
+        place(0, 0, max(k, 1u), false, first, row, sample, lane);
         ++logged;
         size = 1;
     }
 
     // An admitted entry, held by lane j, takes position pos.
-    __device__ __forceinline__ void place(int pos, int j, uint32_t k, uint32_t p, float first,
-                                          uint32_t row, float b, uint32_t sample, int lane)
+    __device__ __forceinline__ void place(int pos, int j, uint32_t k, bool is_unused, float first,
+                                          uint32_t row, uint32_t sample, int lane)
     {
         if (lane == j) {
             entry[pos] = make_uint2(row, sample);
-            if constexpr (kBase) base[pos] = b;
             if (!kNan || !eager)
                 __hip_atomic_store(log + (logged & log_mask),
                                    (static_cast<uint64_t>(static_cast<uint32_t>(pos)) << 32) |
                                        __float_as_uint(first),
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        put(pos, k, p, lane);
+        put(pos, k, is_unused, lane);
     }
 
     // The ordered admission of one step: lane by lane, an entry enters unless
     // the frontier is full and its greatest key is less; past Q entries the
     // greatest leaves.  Returns the lanes admitted.
-    __device__ __forceinline__ uint64_t admit(bool cand, float first, uint32_t row, float b,
+    __device__ __forceinline__ uint64_t admit(bool cand, float first, uint32_t row,
                                               uint32_t sample, int lane)
     {
         if constexpr (kNan) {
@@ -229,7 +238,7 @@ struct SetFrontier {
                 catch_up(lane);
                 eager = true;
             }
-            if (eager) return admit_eager(cand, first, row, b, sample, lane);
+            if (eager) return admit_eager(cand, first, row, sample, lane);
         }
         const uint32_t k = order_key(first);
         uint64_t adm = 0;
@@ -254,7 +263,7 @@ struct SetFrontier {
                     static_for<R>([&](auto i) {
                         if (key[int{i}] == top) {
                             key[int{i}] = 0u;
-                            pick[int{i}] = kDone;
+                            unused &= ~(1u << i);
                         }
                     });
                     top_gone = 0;
@@ -265,7 +274,7 @@ struct SetFrontier {
                 }
                 pos = free_pos(lane);
             }
-            place(pos, j, kj, kj, first, row, b, sample, lane);
+            place(pos, j, kj, true, first, row, sample, lane);
             ++logged;
             adm |= 1ull << j;
             if (moved) find_top();
@@ -274,14 +283,14 @@ struct SetFrontier {
     }
 
     // The same with every admission through the heap.
-    __device__ __forceinline__ uint64_t admit_eager(bool cand, float first, uint32_t row, float b,
+    __device__ __forceinline__ uint64_t admit_eager(bool cand, float first, uint32_t row,
                                                  uint32_t sample, int lane)
     {
         const uint32_t k = order_key(first);
         const bool full = heap_size >= Q + 1;
-        const float thr = full ? heap[2].first : 0.0f;
-        float hmax = heap_size >= 3   ? heap[2].first
-                     : heap_size == 2 ? heap[1].first
+        const float thr = full ? heap.first[2] : 0.0f;
+        float hmax = heap_size >= 3   ? heap.first[2]
+                     : heap_size == 2 ? heap.first[1]
                                       : -__builtin_inff();
         uint64_t adm = 0;
         for (uint64_t m = ballot(cand && !(full && thr < first)); m; m &= m - 1) {
@@ -292,14 +301,14 @@ struct SetFrontier {
             const uint32_t kj = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(k), j));
             const int pos = free_pos(lane);
             p.second = static_cast<uint32_t>(pos);
-            place(pos, j, max(kj, 1u), kj, first, row, b, sample, lane);
+            place(pos, j, max(kj, 1u), true, first, row, sample, lane);
             wave_smmh_insert(heap, heap_size, p, lane);
             hmax = fmaxf(hmax, p.first);
             adm |= 1ull << j;
             if (heap_size >= Q + 2) {
-                const int gone = __builtin_amdgcn_readfirstlane(static_cast<int>(heap[2].second));
+                const int gone = __builtin_amdgcn_readfirstlane(static_cast<int>(heap.second[2]));
                 hmax = wave_smmh_pop_max(heap, heap_size, lane);
-                put(gone, 0u, kDone, lane);
+                put(gone, 0u, false, lane);
             }
         }
         size = heap_size - 1;
@@ -311,11 +320,11 @@ struct SetFrontier {
     {
         for (int s0 = 1; s0 < heap_size; s0 += kWave) {
             const int s = s0 + lane;
-            const uint32_t pos = s < heap_size ? heap[s].second : 0u;
+            const uint32_t pos = s < heap_size ? heap.second[s] : 0u;
             uint32_t p = kDone;
             static_for<R>([&](auto i) {
                 const uint32_t v = static_cast<uint32_t>(
-                    __shfl(static_cast<int>(pick[int{i}]), static_cast<int>(pos & 63u), kWave));
+                    __shfl(static_cast<int>(pick(i, key[int{i}])), static_cast<int>(pos & 63u), kWave));
                 if ((pos >> 6) == static_cast<uint32_t>(i)) p = v;
             });
             const uint64_t m = ballot(s < heap_size && p == mn);
@@ -324,51 +333,33 @@ struct SetFrontier {
         return 0;  // not reached: an unused entry is in the heap
     }
 
-    // The next entry (marked used); false when every entry is used.  With
-    // want_base, min_base is the least base over the entries that were unused
-    // before (the one picked included; FLT_MAX when there is none).
-    __device__ __forceinline__ bool pickup(Entry& out, int lane, bool want_base, float& min_base)
+    // The next entry (marked used); false when every entry is used.
+    __device__ __forceinline__ bool pickup(Entry& out, int lane)
     {
         for (;;) {
-            uint32_t p = pick[0];
-            static_for<R>([&](auto i) { p = min(p, pick[int{i}]); });
+            uint32_t p = kDone;
+            static_for<R>([&](auto i) { p = min(p, pick(i, key[int{i}])); });
             const uint32_t mn = wave_min_u32(p);
             int ties = 0, pos = 0;
             static_for<R>([&](auto r) {
                 constexpr int i = R - 1 - r;
-                const uint64_t at = ballot(pick[int{i}] == mn);
+                const uint64_t at = ballot(pick(i, key[int{i}]) == mn);
                 ties += __popcll(at);
                 if (at) pos = 64 * i + __builtin_ctzll(at);
             });
-            const bool none = mn == kDone;
-            const bool open = top_gone > 0 && (mn == top || (kBase && want_base));
-            if (open || (ties > 1 && !none)) {
-                const bool again = open;
+            if (mn == kDone) return false;
+            const bool open = top_gone > 0 && mn == top;
+            if (open || ties > 1) {
                 if (!kNan || !eager) catch_up(lane);
-                if (again) continue;
+                if (open) continue;
                 pos = first_in_heap(mn, lane);
             }
-            if constexpr (kBase) {
-                if (want_base) {
-                    uint32_t mb = UINT32_MAX;
-                    static_for<R>([&](auto i) {
-                        if (pick[int{i}] != kDone) mb = min(mb, order_key(base[64 * i + lane]));
-                    });
-                    const uint32_t m = wave_min_u32(mb);
-                    min_base = m == UINT32_MAX ? FLT_MAX : order_key_float(m);
-                }
-            }
-            if (none) return false;
             const uint2 rs = entry[pos];
             out.first = order_key_float(mn);
             out.second = rs.x;
             out.sample = rs.y;
             out.base = out.first;
-            if constexpr (kBase) out.base = base[pos];
-            const bool me = lane == (pos & (kWave - 1));
-            static_for<R>([&](auto i) {
-                if ((pos >> 6) == i) pick[int{i}] = me ? kDone : pick[int{i}];
-            });
+            if (lane == (pos & (kWave - 1))) unused &= ~(1u << (pos >> 6));
             return true;
         }
     }

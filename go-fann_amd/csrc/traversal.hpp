@@ -100,6 +100,17 @@ struct PqScorer {
     __device__ int m() const { return kM > 0 ? kM : static_cast<int>(pq_dim); }
     __device__ uint32_t width() const { return kSub > 0 ? static_cast<uint32_t>(kSub) : sub; }
 
+    // The scorer with its launch constants from `k` (a kernel argument) and
+    // this route's state.
+    __device__ __forceinline__ PqScorer with_constants(const PqScorer& k) const
+    {
+        PqScorer r = k;
+        r.table = table;
+        r.query = query;
+        r.qw = qw;
+        return r;
+    }
+
     __device__ void setup(uint32_t q, int lane, unsigned char* lds)
     {
         table = reinterpret_cast<float*>(lds);
@@ -166,15 +177,33 @@ struct PqScorer {
         }
     }
 
+    // The code row of a candidate, requested before it is scored.
+    static constexpr int kPreVecs = kM > 0 && kM % 16 == 0 ? kM / 16 : 0;
+    struct Pre {
+        uint4 w[kPreVecs > 0 ? kPreVecs : 1];
+    };
+    __device__ __forceinline__ void preload(uint32_t sample, bool active, Pre& pre) const
+    {
+        if constexpr (kPreVecs > 0) {
+            const uint4* row = reinterpret_cast<const uint4*>(codes + static_cast<size_t>(sample) * stride);
+#pragma unroll
+            for (int i = 0; i < kPreVecs; ++i) pre.w[i] = active ? row[i] : make_uint4(0, 0, 0, 0);
+        }
+    }
+
     __device__ float score(uint32_t sample, bool active) const
+    {
+        Pre pre;
+        preload(sample, active, pre);
+        return score(sample, active, pre);
+    }
+
+    __device__ float score(uint32_t sample, bool active, const Pre& pre) const
     {
         if (!active) return 0.0f;
         const uint8_t* row = codes + static_cast<size_t>(sample) * stride;
-        if constexpr (kM > 0 && kM % 16 == 0) {
-            uint4 w[kM / 16];
-#pragma unroll
-            for (int i = 0; i < kM / 16; ++i) w[i] = reinterpret_cast<const uint4*>(row)[i];
-            const uint32_t* words = reinterpret_cast<const uint32_t*>(w);
+        if constexpr (kPreVecs > 0) {
+            const uint32_t* words = reinterpret_cast<const uint32_t*>(pre.w);
             float t[16];
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
@@ -339,6 +368,17 @@ struct RabitqScorer {
                        : codes + static_cast<size_t>(sample) * (padded_dim / 8);
     }
 
+    // As PqScorer::with_constants.
+    __device__ __forceinline__ RabitqScorer with_constants(const RabitqScorer& k) const
+    {
+        RabitqScorer r = k;
+        r.planes = planes;
+        r.scale = scale;
+        r.k1 = k1;
+        r.g_row = g_row;
+        return r;
+    }
+
     __device__ void setup(uint32_t q, int lane, unsigned char* lds)
     {
         planes = reinterpret_cast<uint32_t*>(lds);
@@ -422,80 +462,113 @@ struct RabitqScorer {
         return active ? s_ip[rank] : 0;
     }
 
-    // Every lane of the wave calls score (the whole-wave path needs them all).
-    __device__ float score(uint32_t sample, bool active) const
+    // What a candidate's score needs from memory, requested before it is
+    // scored: its factors and anchor, and the first vectors of the row where a
+    // lane (or two) scores it alone.
+    static constexpr int kPreVecs = 2;
+    struct Pre {
+        uint4 c[kPreVecs];
+        uint32_t anchor;
+        float f_add, f_rescale;
+    };
+    // This lane's vectors of a row scored a candidate per lane: with `halves`
+    // lane l counts the first half of lane l's row, lane l + 32 the rest.
+    struct Share {
+        uint32_t sample, begin, end;
+        bool active;
+    };
+    __device__ __forceinline__ Share share(uint32_t sample, bool active, int lane) const
+    {
+        const uint32_t vecs = padded_dim / 128;
+        if (!halves) return Share{sample, 0, vecs, active};
+        const bool hi = lane >= 32;
+        const uint32_t s = swap_wave_halves(sample, lane);
+        const uint64_t am = ballot(active);  // every lane votes (not inside the select)
+        const uint32_t lo = (vecs + 1) / 2;
+        return Share{hi ? s : sample, hi ? lo : 0u, hi ? vecs : lo,
+                     ((am >> (lane & 31)) & 1ull) != 0};
+    }
+    __device__ __forceinline__ bool coop() const
+    {
+        return padded_dim == 4096 || padded_dim == 2048;
+    }
+    __device__ __forceinline__ void preload(uint32_t sample, bool active, Pre& pre) const
     {
         const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
-        const uint32_t vecs = padded_dim / 128;
-        uint32_t anchor = 0;
-        float f_add = 0.0f, f_rescale = 0.0f;
+        pre.anchor = 0;
+        pre.f_add = pre.f_rescale = 0.0f;
         if (active && records) {
             const uint8_t* rec = records + static_cast<size_t>(sample) * record_stride + padded_dim / 8;
             const uint32_t* w = reinterpret_cast<const uint32_t*>(rec);
-            f_add = __uint_as_float(w[0]);
-            f_rescale = __uint_as_float(w[1]);
-            anchor = w[2];
+            pre.f_add = __uint_as_float(w[0]);
+            pre.f_rescale = __uint_as_float(w[1]);
+            pre.anchor = w[2];
         } else if (active) {
-            anchor = anchor_ids[sample];
-            f_add = factors[static_cast<size_t>(sample) * 3];
-            f_rescale = factors[static_cast<size_t>(sample) * 3 + 1];
+            pre.anchor = anchor_ids[sample];
+            pre.f_add = factors[static_cast<size_t>(sample) * 3];
+            pre.f_rescale = factors[static_cast<size_t>(sample) * 3 + 1];
         }
+        if (!coop()) {
+            const Share sh = share(sample, active, lane);
+            const uint4* row = reinterpret_cast<const uint4*>(code_row(sh.sample));
+#pragma unroll
+            for (int i = 0; i < kPreVecs; ++i)
+                pre.c[i] = sh.active && sh.begin + i < sh.end ? row[sh.begin + i] : make_uint4(0, 0, 0, 0);
+        }
+    }
+
+    // Every lane of the wave calls score (the whole-wave path needs them all).
+    __device__ float score(uint32_t sample, bool active) const
+    {
+        Pre pre;
+        preload(sample, active, pre);
+        return score(sample, active, pre);
+    }
+
+    __device__ __forceinline__ float score(uint32_t sample, bool active, const Pre& pre) const
+    {
+        const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+        const uint32_t vecs = padded_dim / 128;
+        // (the anchor's distance is on its way while the bits are counted)
+        const float g = active ? g_row[pre.anchor] : 0.0f;
         int32_t ip;
         if (vecs == 32) {
             ip = ip_coop<2>(sample, active, lane);
         } else if (vecs == 16) {
             ip = ip_coop<1>(sample, active, lane);
-        } else if (halves) {
-            const bool hi = lane >= 32;
-            const uint32_t s = swap_wave_halves(sample, lane);
-            const uint64_t am = ballot(active);  // every lane votes (not inside the select)
-            const bool act = ((am >> (lane & 31)) & 1ull) != 0;
-            const uint32_t lo = (vecs + 1) / 2;
+        } else {
+            const Share sh = share(sample, active, lane);
             int32_t part = 0;
-            if (act) {
-                const uint32_t v_end = hi ? vecs : lo;
-                const uint4* row = reinterpret_cast<const uint4*>(code_row(hi ? s : sample));
+            if (sh.active) {
+                const uint4* row = reinterpret_cast<const uint4*>(code_row(sh.sample));
                 const uint4* planes4 = reinterpret_cast<const uint4*>(planes);
                 uint32_t cnt[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-                for (uint32_t v0 = hi ? lo : 0; v0 < v_end; v0 += kCodeBatch) {
-                    uint4 cb[kCodeBatch];
 #pragma unroll
-                    for (int b = 0; b < kCodeBatch; ++b)
-                        cb[b] = v0 + b < v_end ? row[v0 + b] : make_uint4(0, 0, 0, 0);
+                for (int i = 0; i < kPreVecs; ++i)
+                    if (sh.begin + i < sh.end) count_vec(planes4, vecs, sh.begin + i, pre.c[i], cnt);
+                // further code loads go out kScoreBatch at a time before any is
+                // consumed
+                constexpr int kScoreBatch = 4;
+                for (uint32_t v0 = sh.begin + kPreVecs; v0 < sh.end; v0 += kScoreBatch) {
+                    uint4 cb[kScoreBatch];
 #pragma unroll
-                    for (int b = 0; b < kCodeBatch; ++b) {
-                        if (v0 + b >= v_end) break;
+                    for (int b = 0; b < kScoreBatch; ++b)
+                        cb[b] = v0 + b < sh.end ? row[v0 + b] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+                    for (int b = 0; b < kScoreBatch; ++b) {
+                        if (v0 + b >= sh.end) break;
                         count_vec(planes4, vecs, v0 + b, cb[b], cnt);
                     }
                 }
                 part = combine(cnt);
             }
-            ip = part + static_cast<int32_t>(swap_wave_halves(static_cast<uint32_t>(part), lane));
-        } else {
-            if (!active) return 0.0f;
-            const uint4* row = reinterpret_cast<const uint4*>(code_row(sample));
-            const uint4* planes4 = reinterpret_cast<const uint4*>(planes);
-            uint32_t cnt[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-            // Code loads go out kCodeBatch at a time before any is consumed, so
-            // a row costs ceil(vectors / kCodeBatch) memory round trips, not one
-            // per 16 bytes.
-            for (uint32_t v0 = 0; v0 < vecs; v0 += kCodeBatch) {
-                uint4 cb[kCodeBatch];
-#pragma unroll
-                for (int b = 0; b < kCodeBatch; ++b)
-                    cb[b] = v0 + b < vecs ? row[v0 + b] : make_uint4(0, 0, 0, 0);
-#pragma unroll
-                for (int b = 0; b < kCodeBatch; ++b) {
-                    if (v0 + b >= vecs) break;
-                    count_vec(planes4, vecs, v0 + b, cb[b], cnt);
-                }
-            }
-            ip = combine(cnt);
+            ip = halves ? part + static_cast<int32_t>(swap_wave_halves(static_cast<uint32_t>(part), lane))
+                        : part;
         }
         if (!active) return 0.0f;
         const float short_ip = static_cast<float>(ip) * scale;
         const float t = short_ip + k1;
-        return fmaf(f_rescale, t, f_add + g_row[anchor]);
+        return fmaf(pre.f_rescale, t, pre.f_add + g);
     }
 
     __device__ int32_t ip_int(uint32_t sample) const
@@ -566,8 +639,10 @@ __device__ __forceinline__ void load_node(const TraversalArgs& a, const Scorer& 
 }
 
 template <class Scorer, int kVisited>
-__global__ __launch_bounds__(64, GOFANN_TRAVERSAL_MIN_WAVES) void traversal_kernel(TraversalArgs a, Scorer sc)
+__global__ __launch_bounds__(64, GOFANN_TRAVERSAL_MIN_WAVES) void traversal_kernel(TraversalArgs args, Scorer scorer)
 {
+    const TraversalArgs& a = args;
+    Scorer& sc = scorer;
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ uint32_t s_row[kMaxDegree];
     __shared__ uint32_t s_samp[kMaxDegree];
@@ -660,6 +735,13 @@ __global__ __launch_bounds__(64, GOFANN_TRAVERSAL_MIN_WAVES) void traversal_kern
         // 111 VGPRs, RaBitQ 118-120, no spills; with the lane hoisted out of
         // the loop both reach the 128-VGPR budget and spill)
         const int lane = opaque_lane(wave_lane);
+        // and so are the arguments (step_args: 309-358 scalar registers of the
+        // RaBitQ kernels were spilled into vector lanes, 100-114 are)
+        constexpr uint32_t kScorerAt = (sizeof(TraversalArgs) + alignof(Scorer) - 1) / alignof(Scorer) *
+                                       alignof(Scorer);
+        const TraversalArgs& a = step_args<TraversalArgs>();
+        const Scorer step_sc = scorer.with_constants(step_args<Scorer>(kScorerAt));
+        const Scorer& sc = step_sc;
         const uint32_t now_local = now.second & ~kPoolUsed;
         ++step;
 
@@ -714,6 +796,11 @@ __global__ __launch_bounds__(64, GOFANN_TRAVERSAL_MIN_WAVES) void traversal_kern
         LaneRow lrow;
         uint4 lslab;
         lane_row_bounds(a.pred, my_sample, need_pass, lrow, lslab);
+        // the candidates' code rows, whose lines with records are the slabs':
+        // on their way during the verdict (with the windows of the visited
+        // probe 26.9 -> 25.4 ms, 12,900 routes of 512 bits, Q = 448)
+        typename Scorer::Pre pre;
+        sc.preload(my_sample, keep, pre);
 
         // Verdict of the expanded node (backend_pq.cu:4393-4441).  Skipped
         // when the pool ran dry: the loop leaves below before reading it.
@@ -807,7 +894,7 @@ __global__ __launch_bounds__(64, GOFANN_TRAVERSAL_MIN_WAVES) void traversal_kern
         // entries; predicate pass bits and priorities
         // (backend_pq.cu:4704-4747, 4826-4864).
         if (need_pass) lane_row_fill(a.pred, lrow, my_sample, lslab);
-        const float dist = sc.score(my_sample, keep);
+        const float dist = sc.score(my_sample, keep, pre);
         scored += list_len;
         float first = dist;
         if (keep && bonuses) {
@@ -1031,11 +1118,14 @@ struct Placement {
     int resident;
 };
 
-// Visited-set placement for one scorer configuration.  hash_mode picks it; auto takes the most resident routes per
-// CU, preferring LDS storage on ties (full table, then the spilling table,
-// then the global slab).
+// Visited-set placement for one scorer configuration.  hash_mode picks it;
+// auto takes the full LDS table, else the spilling one, where all `routes` are
+// resident with it (1,200 routes of 4096 bits: 7.84 ms
+// with the global slab, 7.64 so); else the most resident routes per CU, preferring
+// LDS storage on ties (full table, then the spilling table, then the global
+// slab).
 template <class Scorer>
-Placement choose_visited(Context* ctx, const Layout& l, int hash_mode)
+Placement choose_visited(Context* ctx, const Layout& l, int hash_mode, uint32_t routes)
 {
     const Placement full{kVisitedLds, l.bytes(kVisitedLds),
                          resident_per_cu(ctx, traversal_kernel<Scorer, kVisitedLds>,
@@ -1049,6 +1139,11 @@ Placement choose_visited(Context* ctx, const Layout& l, int hash_mode)
     if (hash_mode == GOFANN_PLACE_LDS) return full;
     if (hash_mode == GOFANN_PLACE_GLOBAL) return glob;
     if (hash_mode == GOFANN_PLACE_SPILL) return spill;
+    const auto holds = [&](const Placement& p) {
+        return static_cast<uint64_t>(p.resident) * static_cast<uint64_t>(ctx->compute_units) >= routes;
+    };
+    if (holds(full)) return full;
+    if (holds(spill)) return spill;
     Placement best = full;
     if (spill.resident > best.resident) best = spill;
     if (glob.resident > best.resident) best = glob;
@@ -1134,8 +1229,8 @@ int pq_search_ms(Context* ctx, const gofann_pq_view* pq, const void* queries, in
     const Layout ld = make_layout(DirectScorer::lds_bytes(pq->dim, pq->pq_dim), p->queue_limit,
                                   p->result_width);
     Placement pt{kVisitedGlobal, 0, 0}, pd{kVisitedGlobal, 0, 0};
-    if (p->table_mode != GOFANN_PLACE_GLOBAL) pt = choose_visited<TableScorer>(ctx, lt, p->hash_mode);
-    if (p->table_mode != GOFANN_PLACE_LDS) pd = choose_visited<DirectScorer>(ctx, ld, p->hash_mode);
+    if (p->table_mode != GOFANN_PLACE_GLOBAL) pt = choose_visited<TableScorer>(ctx, lt, p->hash_mode, r->count);
+    if (p->table_mode != GOFANN_PLACE_LDS) pd = choose_visited<DirectScorer>(ctx, ld, p->hash_mode, r->count);
     const bool direct = p->table_mode == GOFANN_PLACE_GLOBAL ||
                         (p->table_mode == GOFANN_PLACE_AUTO && pd.resident > pt.resident);
     ctx->last_table_in_lds = direct ? 0 : 1;
