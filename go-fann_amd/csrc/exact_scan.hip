@@ -9,8 +9,10 @@
 // route the result is the topk least (distance, id) pairs over the distinct
 // listed samples that pass the filter.
 //
-// Here one 256-thread workgroup scans one route in chunks of the 2048-slot
-// LDS pair array (running top-k + chunk):
+// Here one 256-thread workgroup scans one route -- or, where the routes alone
+// would leave the chip part idle, one of up to 16 runs of its rows, whose
+// lists a second kernel merges -- in chunks of the 2048-slot LDS pair array
+// (running top-k + chunk):
 //  * the chunk's valid, predicate-passing samples are compacted into the
 //    chunk slots (order is free: the (distance, id) sort fixes it);
 //  * serial order: a lane per row, the chain in d order, rows read through
@@ -53,9 +55,37 @@ struct ExactScanArgs {
     float* out_dists;
     uint32_t* pass_counts;
     uint32_t tile_offset;  // bytes from the LDS base to the tiles
+    // split: workgroups per route, each with a run of its rows; their lists
+    // [routes][parts][k] and pass counts [routes][parts] before the merge
+    uint32_t parts;
+    float* part_d;
+    uint32_t* part_id;
+    uint32_t* part_pass;
 };
 
 constexpr int kExactScanMaxTopk = 64;
+constexpr uint32_t kExactScanMaxParts = 16;  // parts x k lists fit the merge's pair array
+
+// The first k distinct ids of a sorted list, in place; the slots up to
+// k_pow2 past them are emptied.  One lane.
+__device__ __forceinline__ void keep_distinct(float* d, uint32_t* id, int slots, int k, int k_pow2)
+{
+    int o = 0;
+    uint32_t prev = UINT32_MAX;
+    for (int i = 0; i < slots && o < k; ++i) {
+        const uint32_t v = id[i];
+        if (v == UINT32_MAX) break;
+        if (v == prev) continue;
+        prev = v;
+        d[o] = d[i];
+        id[o] = v;
+        ++o;
+    }
+    for (; o < k_pow2; ++o) {
+        d[o] = __builtin_inff();
+        id[o] = UINT32_MAX;
+    }
+}
 
 // kTile: 0 -- the serial order one thread per row reading its own row (any
 // row length); 16 or 32 -- the serial order through LDS tiles of that many
@@ -71,7 +101,8 @@ __global__ __launch_bounds__(kScanThreads) void exact_scan_kernel(ExactScanArgs 
     __shared__ uint32_t s_n;
     __shared__ uint32_t s_pass;
     const int tid = static_cast<int>(threadIdx.x);
-    const uint32_t route = blockIdx.x;
+    const uint32_t route = blockIdx.x / a.parts;
+    const uint32_t part = blockIdx.x % a.parts;
     if (route >= a.routes) return;
     const float inf = __builtin_inff();
 
@@ -87,8 +118,15 @@ __global__ __launch_bounds__(kScanThreads) void exact_scan_kernel(ExactScanArgs 
     __syncthreads();
 
     const bool enabled = pred_enabled(a.pred, route);
-    const uint32_t begin = a.cand_offsets[route];
-    const uint32_t count = a.cand_sizes[route];
+    uint32_t begin = a.cand_offsets[route];
+    uint32_t count = a.cand_sizes[route];
+    if (a.parts > 1) {  // whole passes of the workgroup's rows per part
+        const uint32_t run = (count / a.parts / kScanThreads + 1u) * kScanThreads;
+        const uint64_t first = static_cast<uint64_t>(run) * part;
+        count = first < count ? count - static_cast<uint32_t>(first) : 0u;
+        count = count < run ? count : run;
+        begin += static_cast<uint32_t>(first);
+    }
     const size_t row_bytes = static_cast<size_t>(a.dim) * elem_bytes(kElem);
     const int chunk = kScanSlots - a.k_pow2;
     uint32_t passes = 0;
@@ -154,39 +192,70 @@ __global__ __launch_bounds__(kScanThreads) void exact_scan_kernel(ExactScanArgs 
                 }
             }
         }
-        for (int i = a.k_pow2 + n + tid; i < kScanSlots; i += kScanThreads) {
+        // sorted: the running list and the chunk, up to the next power of two
+        int slots = 2;
+        while (slots < a.k_pow2 + n) slots <<= 1;
+        for (int i = a.k_pow2 + n + tid; i < slots; i += kScanThreads) {
             s_d[i] = inf;
             s_id[i] = UINT32_MAX;
         }
         __syncthreads();
-        bitonic_sort(s_d, s_id, kScanSlots, tid, kScanThreads);
-        if (tid == 0) {
-            int o = 0;
-            uint32_t prev = UINT32_MAX;
-            for (int i = 0; i < kScanSlots && o < a.k; ++i) {
-                const uint32_t id = s_id[i];
-                if (id == UINT32_MAX) break;
-                if (id == prev) continue;
-                prev = id;
-                s_d[o] = s_d[i];
-                s_id[o] = id;
-                ++o;
-            }
-            for (; o < a.k_pow2; ++o) {
-                s_d[o] = inf;
-                s_id[o] = UINT32_MAX;
-            }
-        }
+        bitonic_sort(s_d, s_id, slots, tid, kScanThreads);
+        if (tid == 0) keep_distinct(s_d, s_id, slots, a.k, a.k_pow2);
         __syncthreads();
     }
     atomicAdd(&s_pass, passes);
     __syncthreads();
+    if (a.parts > 1) {
+        const size_t list = (static_cast<size_t>(route) * a.parts + part) * static_cast<size_t>(a.k);
+        for (int i = tid; i < a.k; i += kScanThreads) {
+            a.part_d[list + i] = s_d[i];
+            a.part_id[list + i] = s_id[i];
+        }
+        if (tid == 0) a.part_pass[static_cast<size_t>(route) * a.parts + part] = s_pass;
+        return;
+    }
     for (int i = tid; i < a.k; i += kScanThreads) {
         const uint32_t id = s_id[i];
         a.out_ids[static_cast<size_t>(route) * a.k + i] = id;
         a.out_dists[static_cast<size_t>(route) * a.k + i] = id == UINT32_MAX ? FLT_MAX : s_d[i];
     }
     if (tid == 0 && a.pass_counts) a.pass_counts[route] = s_pass;
+}
+
+// The route's list from its parts' lists: a sample listed in two parts has
+// the same distance in both, so the same sort and the same dedup apply.
+__global__ __launch_bounds__(kScanThreads) void exact_scan_merge_kernel(ExactScanArgs a)
+{
+    __shared__ float s_d[kScanSlots];
+    __shared__ uint32_t s_id[kScanSlots];
+    const int tid = static_cast<int>(threadIdx.x);
+    const uint32_t route = blockIdx.x;
+    if (route >= a.routes) return;
+    const int n = static_cast<int>(a.parts) * a.k;
+    int slots = 2;
+    while (slots < n || slots < a.k_pow2) slots <<= 1;
+    const size_t list = static_cast<size_t>(route) * static_cast<size_t>(n);
+    for (int i = tid; i < slots; i += kScanThreads) {
+        s_d[i] = i < n ? a.part_d[list + i] : __builtin_inff();
+        s_id[i] = i < n ? a.part_id[list + i] : UINT32_MAX;
+    }
+    __syncthreads();
+    bitonic_sort(s_d, s_id, slots, tid, kScanThreads);
+    if (tid == 0) {
+        keep_distinct(s_d, s_id, slots, a.k, a.k_pow2);
+        if (a.pass_counts) {
+            uint32_t sum = 0;
+            for (uint32_t p = 0; p < a.parts; ++p) sum += a.part_pass[static_cast<size_t>(route) * a.parts + p];
+            a.pass_counts[route] = sum;
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < a.k; i += kScanThreads) {
+        const uint32_t id = s_id[i];
+        a.out_ids[static_cast<size_t>(route) * a.k + i] = id;
+        a.out_dists[static_cast<size_t>(route) * a.k + i] = id == UINT32_MAX ? FLT_MAX : s_d[i];
+    }
 }
 
 namespace {
@@ -205,10 +274,42 @@ int launch_exact_scan(Context* ctx, const ExactScanArgs& a, uint32_t lds)
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) !=
         hipSuccess)
         return ctx->fail_hip("hipFuncSetAttribute exact posting scan");
-    hipLaunchKernelGGL((exact_scan_kernel<kElem, kOrder, kTile>), dim3(a.routes),
+    hipLaunchKernelGGL((exact_scan_kernel<kElem, kOrder, kTile>), dim3(a.routes * a.parts),
                        dim3(kScanThreads), lds, ctx->stream, a);
+    if (a.parts > 1)
+        hipLaunchKernelGGL(exact_scan_merge_kernel, dim3(a.routes), dim3(kScanThreads), 0, ctx->stream, a);
     if (hipGetLastError() != hipSuccess) return ctx->fail_hip("exact posting scan launch");
     return GOFANN_OK;
+}
+
+// Workgroups per route.  About 16 workgroups a CU fill the chip and even out
+// its end (600 routes of 4,000 f32 rows, dim 1024: 2.63 ms with one each, which
+// 256 CUs finish in uneven turns, 1.79 with seven); the lists' lengths are on
+// the device, so every route is cut alike.
+// One where the routes are enough, where the stream is captured (a graph
+// would keep the scratch's address, which a later call may replace) and where
+// there is no memory for the parts.
+uint32_t scan_parts(Context* ctx, ExactScanArgs& a)
+{
+    const uint64_t want = 16ull * static_cast<uint64_t>(ctx->compute_units);
+    uint64_t parts = (want + a.routes - 1) / a.routes;
+    if (parts > kExactScanMaxParts) parts = kExactScanMaxParts;
+    if (parts <= 1) return 1;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return 1;
+    }
+    if (st != hipStreamCaptureStatusNone) return 1;
+    const size_t lists = static_cast<size_t>(a.routes) * parts;
+    const size_t pairs = lists * static_cast<size_t>(a.k);
+    uint32_t* p = static_cast<uint32_t*>(
+        ctx->scratch(Context::kScratchScan, (2 * pairs + lists) * sizeof(uint32_t)));
+    if (!p) return 1;
+    a.part_d = reinterpret_cast<float*>(p);
+    a.part_id = p + pairs;
+    a.part_pass = p + 2 * pairs;
+    return static_cast<uint32_t>(parts);
 }
 
 // Serial order: LDS tiles of 32 words per row where the row allows them and
@@ -277,6 +378,9 @@ int exact_posting_scan(Context* ctx, const void* base, int base_elem, uint32_t d
     a.out_dists = out_dists;
     a.pass_counts = pass_counts;
     a.tile_offset = 0;
+    a.part_d = nullptr;
+    a.part_id = a.part_pass = nullptr;
+    a.parts = scan_parts(ctx, a);
     switch (base_elem) {
     case GOFANN_ELEM_F32:
         return launch_exact_scan_order<GOFANN_ELEM_F32>(ctx, a, lds, fixed, order);

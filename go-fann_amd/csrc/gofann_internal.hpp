@@ -23,7 +23,8 @@ struct Context {
         kScratchRange = 3,  // per-segment range-scan shortlists before the merge
         kScratchBuild = 4,  // index construction (k-means, kNN, graph optimisation)
         kScratchLog = 5,    // admission logs of the set frontier
-        kScratchCount = 6
+        kScratchScan = 6,   // the exact posting scan's lists per part before the merge
+        kScratchCount = 7
     };
 
     int device = 0;

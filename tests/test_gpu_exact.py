@@ -296,6 +296,39 @@ def test_exact_posting_scan_matches_oracle(gpu_ctx, scan_worlds, dim, dtype, ord
             assert (oi[:, 0] != U32MAX).sum() > rs.count // 2
 
 
+@pytest.mark.parametrize("dtype,order", [("u8", _lib.EXACT_ORDER_SERIAL),
+                                         ("f32", _lib.EXACT_ORDER_WARP)])
+def test_exact_posting_scan_split_lists(gpu_ctx, scan_worlds, dtype, order):
+    """Few routes: each list is cut into runs of whole 256-row passes that
+    are merged.  List lengths at the edges of a run and of the number of
+    runs, samples listed in several runs, no candidate in some runs."""
+    dim = 37
+    wl, li = scan_worlds[dim]
+    x = wl.base.numpy()
+    scale = 255.0 / float(x.max() - x.min())
+    rows = lambda t: (np.clip(np.round((t - x.min()) * scale), 0, 255).astype(np.uint8)
+                      if dtype == "u8" else t.astype(np.float32))
+    base, q = rows(x), rows(wl.queries.numpy())
+    sizes = np.array([0, 1, 255, 256, 257, 511, 512, 4095, 4096, 4097, 8191, 9000], np.uint32)
+    offs = np.zeros(len(sizes), np.uint32)
+    offs[1:] = np.cumsum(sizes)[:-1]
+    rng = np.random.default_rng(5)
+    ids = rng.integers(0, base.shape[0], int(sizes.sum())).astype(np.uint32)
+    ids[offs[9]: offs[9] + 4097] = np.arange(4097) % 300     # every run lists the same samples
+    ids[offs[10]: offs[10] + 4096] = U32MAX                  # runs without a candidate
+    ids[offs[11]: offs[11] + 9000] = np.arange(9000) % 3     # fewer samples than k
+    rq = np.arange(len(sizes), dtype=np.uint32)
+    db, dq = torch.from_numpy(base).cuda(), torch.from_numpy(q).cuda()
+    for k in (1, 10, 64):
+        say("exact posting scan split lists", dtype, "order", order, "k", k)
+        oi, od, op = po.exact_posting_scan(None, base, q, rq, ids, offs, sizes, k, order)
+        gi_, gd, gp_ = gs.exact_posting(gpu_ctx, db, dq, rq, ids, offs, sizes, k, order, None)
+        torch.cuda.synchronize()
+        assert np.array_equal(gi_.cpu().numpy().view(np.uint32).reshape(-1, k), oi)
+        assert np.array_equal(gd.cpu().numpy().reshape(-1, k).view(np.uint32), od.view(np.uint32))
+        assert np.array_equal(gp_.cpu().numpy().view(np.uint32), op)
+
+
 def test_exact_search_invalid_seeds(gpu_ctx, eworld):
     wl, li, rs = eworld
     say("exact search invalid seeds")
