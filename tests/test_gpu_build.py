@@ -99,6 +99,26 @@ def test_pq_encode_and_train_match_oracle(hip, dtype, dim, pq_dim):
     assert np.array_equal(gc.cpu().numpy().view(np.uint32), wc.view(np.uint32))
 
 
+@pytest.mark.parametrize("sub", [2, 4, 8, 16])
+def test_pq_encode_least_centre(hip, sub):
+    """The least of 256 centres by groups of 16: the lowest of equal centres
+    in one group and across groups, the first and last of a group, and rows
+    whose every distance is NaN, infinite or (0 is then kept) overflows."""
+    say("pq least centre", sub)
+    rng = np.random.default_rng(sub)
+    c = rng.standard_normal((256, 2 * sub)).astype(np.float32)
+    c[7], c[3] = c[40], c[40]
+    c[255], c[16] = c[200], c[31]
+    c[100] = np.nan
+    c[101] = np.inf
+    x = np.concatenate([c, rng.standard_normal((300, 2 * sub)).astype(np.float32)])
+    x[300], x[301], x[302] = np.nan, np.inf, 3e38
+    want = po.build_pq_encode(x, c, 2)
+    assert want[40, 0] == 3 and want[302, 0] == 0
+    got = hip.pq_encode(hip.rows(torch.from_numpy(x)), torch.from_numpy(c), 2)
+    assert np.array_equal(got.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("dtype", DT)
 def test_kmeans_match_oracle(hip, dtype):
     say("kmeans", dtype.__name__)
