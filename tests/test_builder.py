@@ -72,6 +72,16 @@ def test_navigable_links_hold_the_bucket_knn_prefix():
     assert checked > m // 2
 
 
+@pytest.mark.parametrize("bound,n", [(1, 40), (6, 0), (1 << 16, 900), ((1 << 16) + 1, 900),
+                                     (1 << 32, 900)])
+def test_stable_order(bound, n):
+    """Equal keys keep their order on both sides of the 16-bit line."""
+    rng = np.random.default_rng(n)
+    keys = rng.choice(np.array([0, bound // 2, bound - 1], np.uint32), size=n)
+    assert np.array_equal(gi._stable_order(keys, bound),
+                          np.argsort(keys.astype(np.int64), kind="stable"))
+
+
 def test_train_kmeans_is_seeded_and_deterministic():
     x = torch.from_numpy(np.random.default_rng(4).standard_normal((3000, 8)).astype(np.float32))
     a = gi.train_kmeans(x, 16, iters=5, sample=2000, seed=11, backend=CPU_BUILD)
