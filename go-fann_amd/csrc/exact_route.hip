@@ -223,8 +223,11 @@ static int exact_search_impl(Context* ctx, const void* base, int base_elem, uint
         case GOFANN_ELEM_F16: rc = launch_set<GOFANN_ELEM_F16>(sh, fchunks, regs); break;
         default: rc = launch_set<GOFANN_ELEM_U8>(sh, 0, regs); break;
         }
-        // (below 64 slots the set takes more LDS than the heap)
-        if (rc != GOFANN_ERR_UNSUPPORTED) return rc;
+        // The heap frontier runs where the set takes more LDS than a workgroup
+        // has (below 64 slots it takes more than the heap) or where its rings
+        // leave no memory for the visited slabs.
+        if (rc != GOFANN_ERR_UNSUPPORTED && rc != GOFANN_ERR_NOMEM) return rc;
+        if (rc == GOFANN_ERR_NOMEM) ctx->release(Context::kScratchLog);
     }
     const int chunks = (GOFANN_EXACT_FIXED_ROWS && (dim == 128 || dim == 192 || dim == 256))
                            ? static_cast<int>(dim / 16)

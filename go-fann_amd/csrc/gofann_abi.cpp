@@ -32,6 +32,14 @@ void* Context::scratch(int slot, size_t bytes)
     return p;
 }
 
+void Context::release(int slot)
+{
+    if (scratch_ptr[slot] == nullptr || hipStreamSynchronize(stream) != hipSuccess) return;
+    (void)hipFree(scratch_ptr[slot]);
+    scratch_ptr[slot] = nullptr;
+    scratch_bytes[slot] = 0;
+}
+
 }  // namespace gofann
 
 using gofann::Context;

@@ -56,6 +56,8 @@ struct Context {
     // Returns a device buffer of at least `bytes` for `slot` (grows, never
     // shrinks; freed by gofann_destroy).  nullptr on allocation failure.
     void* scratch(int slot, size_t bytes);
+    // Frees `slot`'s buffer, once the stream is done with it.
+    void release(int slot);
 };
 
 int pq_search(Context* ctx, const gofann_pq_view* pq, const void* queries, int query_elem,

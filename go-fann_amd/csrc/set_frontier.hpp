@@ -370,6 +370,10 @@ struct SetFrontier {
 // Q = 72 and 1260 at Q = 416.
 inline uint32_t set_log_entries(int q) { return q <= 112 ? 1024u : 2048u; }
 
+// The context keeps its rings from call to call; a launch of more routes
+// (131,072 at Q > 112) takes the heap frontier.
+constexpr size_t kSetLogBytes = size_t{2} << 30;
+
 // Registers a lane for a beam of q, with the log rings of `routes` launch
 // slots, or 0 where the heap frontier runs instead: beams that the wave heap
 // operations do not hold, streams under capture (the graph would keep the
@@ -388,8 +392,9 @@ inline int set_registers(Context* ctx, int q, uint32_t routes, uint64_t** log)
         return 0;
     }
     if (st != hipStreamCaptureStatusNone) return 0;
-    *log = static_cast<uint64_t*>(ctx->scratch(
-        Context::kScratchLog, static_cast<size_t>(routes) * set_log_entries(q) * sizeof(uint64_t)));
+    const size_t bytes = static_cast<size_t>(routes) * set_log_entries(q) * sizeof(uint64_t);
+    if (bytes > kSetLogBytes) return 0;
+    *log = static_cast<uint64_t*>(ctx->scratch(Context::kScratchLog, bytes));
     return *log != nullptr ? regs : 0;
 }
 

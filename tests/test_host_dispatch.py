@@ -1,0 +1,135 @@
+"""Host side of the launches on a machine without a GPU: which kernel a call
+takes, what it allocates and what it refuses.
+
+The library is loaded over a stand-in for the HIP runtime (fake_hip.cpp),
+which records launches instead of running them, in a process of its own: the
+file runs itself with the case's name.  256 CUs of 160 KB LDS, 16 resident
+one-wave workgroups a CU."""
+from __future__ import annotations
+
+import ctypes as C
+import importlib.util
+import os
+import re
+import shutil
+import subprocess
+import sys
+from pathlib import Path
+
+ROOT = Path(__file__).resolve().parent.parent
+LIB = ROOT / "go-fann_amd" / "libgofann_hip.so"
+
+GIB = 1 << 30
+SIDE = 0x1000  # a stream that is not the default one
+
+
+class Fake:
+    """The library over the stand-in runtime."""
+
+    def __init__(self, stub: str):
+        self.hip = C.CDLL(stub, mode=os.RTLD_NOW | os.RTLD_GLOBAL)
+        self.hip.fake_limit.argtypes = [C.c_size_t]
+        self.hip.fake_used.restype = C.c_size_t
+        self.hip.fake_name.restype = C.c_char_p
+        self.hip.fake_capture.argtypes = [C.c_void_p]
+        spec = importlib.util.spec_from_file_location(
+            "_lib", ROOT / "go-fann_amd" / "gofann_amd" / "_lib.py")
+        self.L = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(self.L)
+        self.lib = self.L.load()
+        self.mem = C.create_string_buffer(1 << 20)  # what every "device array" points to
+        self.p = (C.addressof(self.mem) + 255) & ~255
+
+    def context(self, stream=0):
+        h = self.L.P()
+        assert self.lib.gofann_create(0, C.byref(h)) == 0
+        assert self.lib.gofann_set_stream(h, self.L.P(stream)) == 0
+        return h
+
+    def launched(self):
+        """Names and grids of the launches since the last call."""
+        out = [(self.hip.fake_name(i).decode(), self.hip.fake_grid(i))
+               for i in range(self.hip.fake_launches())]
+        self.hip.fake_clear()
+        return out
+
+    def graph(self, degree=32):
+        L, p = self.L, self.p
+        return L.GraphView(p, p, p, 1000, degree, 1, 1000, None)
+
+    def routes(self, count):
+        p = self.p
+        return self.L.Routes(p, p, p, None, None, None, None, None, None, 0, count, None)
+
+    def exact(self, ctx, elem, dim, beam, count, place=0):
+        L, p = self.L, self.p
+        return self.lib.gofann_exact_search(ctx, p, elem, dim, 1000, p, self.graph(), None,
+                                            L.PredicateView(), self.routes(count),
+                                            L.ExactParams(beam, 1, 2, 0, 10, place), p, p, None)
+
+
+def exact_kernel(name: str):
+    """(visited placement, set registers) of an exact-route kernel's name."""
+    m = re.search(r"exact_(route|set)_kernelILi(\d)ELin?\d+ELi\d+E(?:Li(\d)E)?E", name)
+    assert m, name
+    return {0: "global", 1: "lds", 2: "spill"}[int(m.group(2))], int(m.group(3) or 0)
+
+
+# --------------------------------------------------------------------------
+# Cases (run in the child process)
+# --------------------------------------------------------------------------
+def case_rings_without_slabs(f: Fake):
+    """20,000 f32 routes whose rings fit in memory and whose visited slabs
+    then do not: the heap frontier takes them, and the rings are given back."""
+    ctx = f.context()
+    slabs, rings = 20_000 * 16384, 20_000 * 2048 * 8
+    f.hip.fake_limit(f.hip.fake_used() + rings + slabs // 2)
+    assert f.exact(ctx, f.L.ELEM_F32, 64, 300, 20_000) == f.L.OK
+    [(name, grid)] = f.launched()
+    assert exact_kernel(name)[1] == 0 and grid == 20_000
+    assert f.hip.fake_used() <= slabs + 1024
+    # with room for both, the set frontier
+    f.hip.fake_limit(8 * GIB)
+    assert f.exact(ctx, f.L.ELEM_F32, 64, 300, 20_000) == f.L.OK
+    [(name, _)] = f.launched()
+    assert exact_kernel(name)[1] == 8
+
+
+def case_rings_are_bounded(f: Fake):
+    """A launch whose rings would pass 2 GiB takes the heap frontier."""
+    ctx = f.context()
+    for count, regs in ((1 << 17, 8), ((1 << 17) + 1, 0)):
+        assert f.exact(ctx, f.L.ELEM_F16, 64, 300, count) == f.L.OK
+        [(name, _)] = f.launched()
+        assert exact_kernel(name)[1] == regs
+
+
+# --------------------------------------------------------------------------
+CASES = sorted(k[5:] for k in globals() if k.startswith("case_"))
+
+
+def pytest_generate_tests(metafunc):
+    if "case" in metafunc.fixturenames:
+        metafunc.parametrize("case", CASES)
+
+
+def _stub(tmp: Path) -> Path:
+    out = tmp / "libfake_hip.so"
+    if not out.exists():
+        cxx = shutil.which("g++") or "g++"
+        subprocess.run([cxx, "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                        "-I/opt/rocm/include", str(ROOT / "tests" / "fake_hip.cpp"),
+                        "-o", str(out)], check=True, timeout=300)
+    return out
+
+
+def test_dispatch(case, hip_lib_path, tmp_path_factory):
+    base = tmp_path_factory.getbasetemp() / "fake_hip"
+    base.mkdir(exist_ok=True)
+    res = subprocess.run([sys.executable, __file__, case, str(_stub(base))], timeout=120,
+                         capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout[-2000:] + res.stderr[-2000:]
+
+
+if __name__ == "__main__":
+    globals()["case_" + sys.argv[1]](Fake(sys.argv[2]))
