@@ -286,25 +286,18 @@ int launch_exact_scan(Context* ctx, const ExactScanArgs& a, uint32_t lds)
 // its end (600 routes of 4,000 f32 rows, dim 1024: 2.63 ms with one each, which
 // 256 CUs finish in uneven turns, 1.79 with seven); the lists' lengths are on
 // the device, so every route is cut alike.
-// One where the routes are enough, where the stream is captured (a graph
-// would keep the scratch's address, which a later call may replace) and where
-// there is no memory for the parts.
+// One where the routes are enough and where there is no buffer for the parts
+// (optional_scratch).
 uint32_t scan_parts(Context* ctx, ExactScanArgs& a)
 {
     const uint64_t want = 16ull * static_cast<uint64_t>(ctx->compute_units);
     uint64_t parts = (want + a.routes - 1) / a.routes;
     if (parts > kExactScanMaxParts) parts = kExactScanMaxParts;
     if (parts <= 1) return 1;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
-        (void)hipGetLastError();
-        return 1;
-    }
-    if (st != hipStreamCaptureStatusNone) return 1;
     const size_t lists = static_cast<size_t>(a.routes) * parts;
     const size_t pairs = lists * static_cast<size_t>(a.k);
     uint32_t* p = static_cast<uint32_t*>(
-        ctx->scratch(Context::kScratchScan, (2 * pairs + lists) * sizeof(uint32_t)));
+        ctx->optional_scratch(Context::kScratchScan, (2 * pairs + lists) * sizeof(uint32_t)));
     if (!p) return 1;
     a.part_d = reinterpret_cast<float*>(p);
     a.part_id = p + pairs;

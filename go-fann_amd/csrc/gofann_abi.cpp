@@ -32,6 +32,24 @@ void* Context::scratch(int slot, size_t bytes)
     return p;
 }
 
+void* Context::optional_scratch(int slot, size_t bytes)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (st != hipStreamCaptureStatusNone) return nullptr;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    void* p = scratch(slot, bytes);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return p;
+}
+
 void Context::release(int slot)
 {
     if (scratch_ptr[slot] == nullptr || hipStreamSynchronize(stream) != hipSuccess) return;

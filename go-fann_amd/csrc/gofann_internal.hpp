@@ -56,6 +56,11 @@ struct Context {
     // Returns a device buffer of at least `bytes` for `slot` (grows, never
     // shrinks; freed by gofann_destroy).  nullptr on allocation failure.
     void* scratch(int slot, size_t bytes);
+    // The same for a buffer that a launch can do without.  nullptr also where
+    // the stream is captured (the graph would keep an address that a later
+    // call may replace); another stream's capture is left intact, which an
+    // allocation in the default capture mode would break.
+    void* optional_scratch(int slot, size_t bytes);
     // Frees `slot`'s buffer, once the stream is done with it.
     void release(int slot);
 };

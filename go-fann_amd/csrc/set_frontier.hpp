@@ -376,9 +376,7 @@ constexpr size_t kSetLogBytes = size_t{2} << 30;
 
 // Registers a lane for a beam of q, with the log rings of `routes` launch
 // slots, or 0 where the heap frontier runs instead: beams that the wave heap
-// operations do not hold, streams under capture (the graph would keep the
-// address of a scratch buffer that a later call may replace), or no memory
-// for the rings.
+// operations do not hold, or no buffer for the rings (optional_scratch).
 inline int set_registers(Context* ctx, int q, uint32_t routes, uint64_t** log)
 {
     const int regs = q + static_cast<int>(kSetSlack) <= 128   ? 2
@@ -386,15 +384,9 @@ inline int set_registers(Context* ctx, int q, uint32_t routes, uint64_t** log)
                      : q + static_cast<int>(kSetSlack) <= 512 ? 8
                                                               : 0;
     if (regs == 0) return 0;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
-    }
-    if (st != hipStreamCaptureStatusNone) return 0;
     const size_t bytes = static_cast<size_t>(routes) * set_log_entries(q) * sizeof(uint64_t);
     if (bytes > kSetLogBytes) return 0;
-    *log = static_cast<uint64_t*>(ctx->scratch(Context::kScratchLog, bytes));
+    *log = static_cast<uint64_t*>(ctx->optional_scratch(Context::kScratchLog, bytes));
     return *log != nullptr ? regs : 0;
 }
 

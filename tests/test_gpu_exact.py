@@ -452,3 +452,42 @@ def test_exact_search_log_ring_wraps(gpu_ctx, eworld):
             a, b = _run_both(gpu_ctx, li, part, base, q, Q, 1)
             for x, y in zip(a, b):
                 assert np.array_equal(x, y)
+
+
+def test_exact_scan_beside_a_capture(gpu_ctx, scan_worlds):
+    """A context's first scan, which allocates its part lists, while torch
+    captures a graph on another stream: both complete."""
+    wl, _ = scan_worlds[128]
+    say("exact posting scan beside a capture")
+    base, q = wl.base.float().cuda(), wl.queries.float().cuda()
+    n = int(q.shape[0])
+    ids = np.random.default_rng(8).integers(0, wl.n, n * 900).astype(np.uint32)
+    offs, sizes = np.arange(n, dtype=np.uint32) * 900, np.full(n, 900, np.uint32)
+    rq = np.arange(n, dtype=np.uint32)
+    want = po.exact_posting_scan(None, wl.base.float().numpy(), wl.queries.float().numpy(), rq, ids,
+                                 offs, sizes, 10, _lib.EXACT_ORDER_SERIAL)
+    dev = [gs.u32(a) for a in (rq, ids, offs, sizes)]
+    out = [torch.zeros(n * 10, dtype=torch.int32, device="cuda"), torch.zeros(n * 10, device="cuda"),
+           torch.zeros(n, dtype=torch.int32, device="cuda")]
+    ctx = _lib.Context(0)
+    side, cap, graph = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    ctx.bind_stream(side)
+    x = torch.zeros(64, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(cap):
+        graph.capture_begin()
+        x.add_(1.0)
+        ctx.check(ctx.lib.gofann_exact_posting_scan(
+            ctx.handle, _lib.ptr(base), _lib.ELEM_F32, 128, wl.n, _lib.ptr(q),
+            _lib.PredicateView(), *[_lib.ptr(t) for t in dev], n, 10, _lib.EXACT_ORDER_SERIAL,
+            *[_lib.ptr(t) for t in out]))
+        graph.capture_end()
+    side.synchronize()
+    for step in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert x.cpu().tolist() == [step + 1.0] * 64
+    assert np.array_equal(out[0].cpu().numpy().view(np.uint32).reshape(n, 10), want[0])
+    assert np.array_equal(out[1].cpu().numpy().reshape(n, 10).view(np.uint32),
+                          want[1].view(np.uint32))
+    ctx.close()

@@ -67,6 +67,12 @@ class Fake:
                                             L.PredicateView(), self.routes(count),
                                             L.ExactParams(beam, 1, 2, 0, 10, place), p, p, None)
 
+    def exact_scan(self, ctx, routes):
+        p = self.p
+        return self.lib.gofann_exact_posting_scan(
+            ctx, p, self.L.ELEM_F32, 64, 1000, p, self.L.PredicateView(), p, p, p, p, routes, 10,
+            self.L.EXACT_ORDER_SERIAL, p, p, None)
+
 
 def exact_kernel(name: str):
     """(visited placement, set registers) of an exact-route kernel's name."""
@@ -102,6 +108,35 @@ def case_rings_are_bounded(f: Fake):
         assert f.exact(ctx, f.L.ELEM_F16, 64, 300, count) == f.L.OK
         [(name, _)] = f.launched()
         assert exact_kernel(name)[1] == regs
+
+
+def case_capture_elsewhere(f: Fake):
+    """A search or a scan that allocates its optional buffers while another
+    stream is captured leaves that capture intact."""
+    for call in (lambda h: f.exact(h, f.L.ELEM_F32, 64, 96, 8, f.L.PLACE_LDS),
+                 lambda h: f.exact_scan(h, 8)):
+        f.hip.fake_capture(0x2000)
+        assert call(f.context(SIDE)) == f.L.OK
+        assert not f.hip.fake_capture_broken()
+        f.hip.fake_capture(None)
+
+
+def case_captured_launches_keep_no_scratch(f: Fake):
+    """Under capture neither allocates: the heap frontier, and one workgroup
+    a route."""
+    f.hip.fake_capture(SIDE)
+    h, used = f.context(SIDE), f.hip.fake_used()
+    assert f.exact(h, f.L.ELEM_F32, 64, 96, 8, f.L.PLACE_LDS) == f.L.OK
+    [(name, _)] = f.launched()
+    assert exact_kernel(name) == ("lds", 0)
+    assert f.exact_scan(h, 8) == f.L.OK
+    [(name, grid)] = f.launched()
+    assert "exact_scan_kernel" in name and grid == 8
+    assert f.hip.fake_used() == used and not f.hip.fake_capture_broken()
+    f.hip.fake_capture(None)
+    # outside it: 16 runs a route and their merge
+    assert f.exact_scan(h, 8) == f.L.OK
+    assert [g for _, g in f.launched()] == [128, 8]
 
 
 # --------------------------------------------------------------------------
