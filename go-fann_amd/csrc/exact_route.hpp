@@ -691,11 +691,33 @@ int exact_resident(Context* ctx, uint32_t lds)
 }
 
 
-// Visited-set placement, then the launch.  Auto: the full LDS table, else the
-// spilling one, where every route of the launch is resident with it; else the
-// most resident routes per CU, the global slab only where it holds a quarter
-// more of them (u8, Q = 72, 57,000 routes: 28 a CU with the slab took 12.15 ms,
-// 24 with the spilling table 12.11).
+// Whether the visited slabs' memory traffic (16 KB a route) is felt: u8
+// launches of more than one round of resident routes whose sets mostly stay
+// within the spilling table (Q <= 72), and of more than two rounds where
+// the rows' own traffic is high (degree x dim of 8 KB a step or more).  The
+// spilling table (23-24 routes a CU) against the slab (28), ms at dim x degree:
+//   192 x 64, Q = 72: 5,000 routes 2.07 / 1.99, 20,000 5.02 / 5.68, 57,000
+//     11.7 / 14.2; Q = 96: 2.53 / 2.43, 6.77 / 7.13, 16.5 / 17.8; 12,000 at
+//     Q = 112 4.36 / 4.07
+//   96 x 32, Q = 64: 6,000 1.84 / 1.81, 45,000 8.13 / 8.34; Q = 96: 2.94 /
+//     2.38, 12.5 / 11.5
+//   96 x 64, Q = 96: 12,000 4.43 / 3.84, 45,000 12.1 / 12.1; 128 x 48: 45,000
+//     12.0 / 11.0
+// (f16 rows, dim 512, Q = 416, 12 against 16 a CU: 12.4 / 10.9; f32 rows of 16 KB,
+// Q = 352, 6 against 7: 186 / 181.)
+template <int kElem>
+bool slabs_cost(const Context* ctx, const ExactArgs& a, uint32_t count, int residents)
+{
+    if (kElem != GOFANN_ELEM_U8) return false;
+    const uint64_t round = static_cast<uint64_t>(residents) * static_cast<uint64_t>(ctx->compute_units);
+    if (a.params.queue_limit <= 72) return count > round;
+    return count > 2 * round && static_cast<uint64_t>(a.dim) * a.graph.degree >= 8192;
+}
+
+// Visited-set placement, then the launch.  Auto: the full LDS table where
+// full_table says so, else the most resident routes per CU, LDS preferred on
+// ties; where the slabs' traffic costs more than residents gain
+// (slabs_cost), the global slab has to hold a quarter more of them.
 // fixed_slab: visited slabs for a placement outside LDS, holding at most
 // fixed_routes routes (the no-alloc entry point); nullptr: context scratch.
 template <int kC, int kElem, int kR>
@@ -715,15 +737,12 @@ int launch_exact(Context* ctx, ExactArgs& a, int hash_mode, uint32_t lds_full,
         mode = kVisitedSpill;
         res = rs;
     } else if (hash_mode == GOFANN_PLACE_AUTO) {
-        const auto holds = [&](int r) {
-            return static_cast<uint64_t>(r) * static_cast<uint64_t>(ctx->compute_units) >= count;
-        };
-        if (!holds(rf)) {
+        if (!full_table(ctx, count, lds_full, rf)) {
             if (rs > res) {
                 mode = kVisitedSpill;
                 res = rs;
             }
-            if (!holds(rs) && rg > res + res / 4) {
+            if (rg > res + (slabs_cost<kElem>(ctx, a, count, rg) ? res / 4 : 0)) {
                 mode = kVisitedGlobal;
                 res = rg;
             }

@@ -65,6 +65,28 @@ struct Context {
     void release(int slot);
 };
 
+// Whether a launch of one wave64 per route keeps every visited set in a full LDS
+// table of its own (`lds` bytes a route, `resident` routes a CU), whatever
+// placement holds the most routes a CU: such routes run 3-7% faster, but their
+// LDS is lost to kernels beside them.  Beside a label-posting scan on another
+// stream, with the full table / the most resident placement, at routes a CU:
+// RaBitQ 512 bits, Q = 64: 1 at 4.70 / 4.62 ms, 2 at 4.71 / 4.67, 4 at 5.03 /
+// 4.75; Q = 384: 1 at 5.29 / 5.29, 2 (49 KB a CU) at 6.10 / 5.35; 4096 bits: 2
+// (56 KB) at 8.81 / 8.21, 4.7 at 12.77 / 9.16; exact f32: 2 at 4.42 / 4.42, 3
+// (55 KB) at 4.58 / 4.43; exact u8: 2 at 4.43 / 4.42, 3 at 4.57 / 4.43.  Alone
+// the same launches gain: 4096 bits at 4.7 a CU 7.44 -> 7.17, exact u8 at 5
+// 1.06 -> 0.99.
+// So a launch on the default stream takes it where all its routes are
+// resident, and one on a stream of the caller's, which is there to run beside
+// others, only up to a quarter of the LDS.
+inline bool full_table(const Context* ctx, uint32_t routes, uint32_t lds, int resident)
+{
+    const uint64_t cus = static_cast<uint64_t>(ctx->compute_units);
+    if (static_cast<uint64_t>(resident) * cus < routes) return false;
+    return ctx->stream == nullptr ||
+           (routes + cus - 1) / cus * lds <= static_cast<uint64_t>(ctx->lds_per_cu) / 4;
+}
+
 int pq_search(Context* ctx, const gofann_pq_view* pq, const void* queries, int query_elem,
               const gofann_graph_view* g, const gofann_predicate_view* pred,
               const gofann_routes* r, const gofann_search_params* p, uint32_t* out_ids,

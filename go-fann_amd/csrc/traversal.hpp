@@ -1119,11 +1119,10 @@ struct Placement {
 };
 
 // Visited-set placement for one scorer configuration.  hash_mode picks it;
-// auto takes the full LDS table, else the spilling one, where all `routes` are
-// resident with it (1,200 routes of 4096 bits: 7.84 ms
-// with the global slab, 7.64 so); else the most resident routes per CU, preferring
-// LDS storage on ties (full table, then the spilling table, then the global
-// slab).
+// auto takes the full LDS table where full_table says so (1,200 routes of 4096
+// bits: 7.63 ms, 7.90 with the global slab, 8.10 with the spilling table), else
+// the most resident routes per CU, preferring LDS storage on ties (full
+// table, then the spilling table, then the global slab).
 template <class Scorer>
 Placement choose_visited(Context* ctx, const Layout& l, int hash_mode, uint32_t routes)
 {
@@ -1139,11 +1138,7 @@ Placement choose_visited(Context* ctx, const Layout& l, int hash_mode, uint32_t 
     if (hash_mode == GOFANN_PLACE_LDS) return full;
     if (hash_mode == GOFANN_PLACE_GLOBAL) return glob;
     if (hash_mode == GOFANN_PLACE_SPILL) return spill;
-    const auto holds = [&](const Placement& p) {
-        return static_cast<uint64_t>(p.resident) * static_cast<uint64_t>(ctx->compute_units) >= routes;
-    };
-    if (holds(full)) return full;
-    if (holds(spill)) return spill;
+    if (full_table(ctx, routes, full.lds, full.resident)) return full;
     Placement best = full;
     if (spill.resident > best.resident) best = spill;
     if (glob.resident > best.resident) best = glob;

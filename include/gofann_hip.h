@@ -175,7 +175,11 @@ typedef struct {
      * hash_mode (visited set): 0 auto, 1 the 4096-slot table in LDS, 2 the
      * same table in a per-route global slab, 3 a 1024-slot LDS table moved
      * into the global slab before it passes 3/4 load.
-     * Auto picks the placement with the most resident routes per CU. */
+     * Auto: a launch whose routes are all resident with the table in LDS takes
+     * it, on a stream other than the default one only up to a quarter of the
+     * LDS; other launches take the placement with the most resident routes per
+     * CU (exact route, large u8 launches: the slab only if it holds a quarter
+     * more than the spilling table). */
     int table_mode;
     int hash_mode;
 } gofann_search_params;

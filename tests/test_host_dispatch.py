@@ -73,6 +73,20 @@ class Fake:
             ctx, p, self.L.ELEM_F32, 64, 1000, p, self.L.PredicateView(), p, p, p, p, routes, 10,
             self.L.EXACT_ORDER_SERIAL, p, p, None)
 
+    def rabitq(self, ctx, bits, beam, count):
+        L, p = self.L, self.p
+        rq = L.RabitqView(p, p, p, p, bits, bits, 64, 1000, None, 0)
+        prm = L.SearchParams(beam, 1, 2, 0, 10, 100, 0.0, 0.0, 0, 0, 0, 0)
+        return self.lib.gofann_rabitq_search(ctx, rq, L.RabitqQueries(p, p, p, p, p, 16),
+                                             self.graph(), L.PredicateView(), self.routes(count),
+                                             prm, p, p, None)
+
+    def placement(self, ctx):
+        """(PQ table in LDS, visited placement) of the last launch."""
+        v = [C.c_int() for _ in range(4)]
+        assert self.lib.gofann_last_placement(ctx, *[C.byref(x) for x in v]) == 0
+        return v[0].value, ("global", "lds", "spill")[v[1].value]
+
 
 def exact_kernel(name: str):
     """(visited placement, set registers) of an exact-route kernel's name."""
@@ -137,6 +151,57 @@ def case_captured_launches_keep_no_scratch(f: Fake):
     # outside it: 16 runs a route and their merge
     assert f.exact_scan(h, 8) == f.L.OK
     assert [g for _, g in f.launched()] == [128, 8]
+
+
+def case_full_table_beside_others(f: Fake):
+    """The full LDS table: every resident launch on the default stream; up to
+    a quarter of a CU's LDS on a stream that may run beside others."""
+    for stream, per_cu, want in ((0, 1, "lds"), (0, 5, "lds"), (SIDE, 1, "lds"),
+                                 (SIDE, 2, "lds"), (SIDE, 3, "spill"), (SIDE, 5, "spill")):
+        h = f.context(stream)
+        assert f.exact(h, f.L.ELEM_F32, 64, 64, per_cu * 256) == f.L.OK
+        assert f.placement(h)[1] == want, (stream, per_cu)
+        assert f.rabitq(h, 512, 64, per_cu * 256) == f.L.OK
+        assert f.placement(h)[1] == want, (stream, per_cu)
+        # 28 KB a route (4096 bits, Q = 320): one a CU
+        assert f.rabitq(h, 4096, 320, per_cu * 256) == f.L.OK
+        want = "lds" if stream == 0 or per_cu == 1 else "global"
+        assert f.placement(h)[1] == want, (stream, per_cu)
+
+
+def case_most_residents(f: Fake):
+    """Past the full table, the most resident routes a CU, also where the
+    spilling table holds the whole launch."""
+    h = f.context()
+    assert f.rabitq(h, 512, 384, 2584) == f.L.OK      # spill 13 a CU, slab 16
+    assert f.placement(h)[1] == "global"
+    assert f.exact(h, f.L.ELEM_F16, 512, 416, 2584) == f.L.OK
+    assert f.placement(h)[1] == "global"
+    # 16 KB rows: 6 with the spilling table, 7 with the slab
+    assert f.exact(h, f.L.ELEM_F32, 4096, 352, 3333) == f.L.OK
+    assert f.placement(h)[1] == "global"
+
+
+def case_u8_slabs(f: Fake):
+    """u8 rows, 24 a CU with the spilling table and 28 with the slab: the
+    slab up to a round (Q <= 72) or two of residents, or where a step reads
+    less than 8 KB of rows."""
+    f.hip.fake_waves(28)
+    h, round_ = f.context(), 28 * 256
+
+    def placed(dim, degree, beam, count):
+        L, p = f.L, f.p
+        assert f.lib.gofann_exact_search(
+            h, p, L.ELEM_U8, dim, 1000, p, f.graph(degree), None, L.PredicateView(),
+            f.routes(count), L.ExactParams(beam, 1, 2, 0, 10, 0), p, p, None) == L.OK
+        return f.placement(h)[1]
+    # (the rows' LDS pads the spilling table to 24 a CU)
+    for dim, degree, beam, count, want in (
+            (1344, 8, 72, round_, "global"), (1344, 8, 72, round_ + 1, "spill"),
+            (1344, 8, 73, 2 * round_, "global"), (1344, 8, 73, 2 * round_ + 1, "spill"),
+            (1344, 6, 73, 2 * round_ + 1, "global"), (1344, 6, 72, round_ + 1, "spill"),
+            (192, 64, 300, 60_000, "global")):
+        assert placed(dim, degree, beam, count) == want, (dim, degree, beam, count)
 
 
 # --------------------------------------------------------------------------
