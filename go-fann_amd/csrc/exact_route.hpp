@@ -675,21 +675,9 @@ constexpr auto exact_kernel()
 template <int kVisited, int kC, int kElem, int kR>
 int exact_resident(Context* ctx, uint32_t lds)
 {
-    if (lds > static_cast<uint32_t>(ctx->lds_per_block)) return 0;
-    const void* k = reinterpret_cast<const void*>(exact_kernel<kVisited, kC, kElem, kR>());
-    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            static_cast<int>(lds)) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
-    }
-    int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, kWave, lds) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
-    }
-    return blocks;
+    return resident_blocks(
+        ctx, reinterpret_cast<const void*>(exact_kernel<kVisited, kC, kElem, kR>()), lds);
 }
-
 
 // Whether the visited slabs' memory traffic (16 KB a route) is felt: u8
 // launches of more than one round of resident routes whose sets mostly stay

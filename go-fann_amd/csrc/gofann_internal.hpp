@@ -65,6 +65,10 @@ struct Context {
     void release(int slot);
 };
 
+// Workgroups of one wave64 with `lds` bytes of dynamic LDS that a CU holds
+// (registers, LDS and wave slots counted); 0 where none fits.
+int resident_blocks(Context* ctx, const void* kernel, uint32_t lds);
+
 // Whether a launch of one wave64 per route keeps every visited set in a full LDS
 // table of its own (`lds` bytes a route, `resident` routes a CU), whatever
 // placement holds the most routes a CU: such routes run 3-7% faster, but their

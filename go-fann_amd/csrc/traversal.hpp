@@ -1091,25 +1091,11 @@ inline int check_params(Context* ctx, const gofann_graph_view* g, const gofann_r
     return GOFANN_OK;
 }
 
-// Resident workgroups per CU of a one-wave traversal launch with `lds`
-// bytes of dynamic LDS (registers, LDS and wave slots all counted).
+// resident_blocks of a traversal kernel.
 template <class Kernel>
 int resident_per_cu(Context* ctx, Kernel kern, uint32_t lds)
 {
-    if (lds > static_cast<uint32_t>(ctx->lds_per_block)) return 0;
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                            static_cast<int>(lds)) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
-    }
-    int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(kern),
-                                                     kWave, lds) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
-    }
-    return blocks;
+    return resident_blocks(ctx, reinterpret_cast<const void*>(kern), lds);
 }
 
 struct Placement {

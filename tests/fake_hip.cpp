@@ -122,6 +122,11 @@ hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int)
     return hipSuccess;
 }
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipFuncGetAttributes(hipFuncAttributes* a, const void*)
+{
+    std::memset(static_cast<void*>(a), 0, sizeof(*a));
+    return hipSuccess;
+}
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* blocks, const void*, int, size_t lds)
 {
     *blocks = std::min<int>(g_waves, lds ? static_cast<int>(kLds / lds) : g_waves);

@@ -182,8 +182,19 @@ def case_most_residents(f: Fake):
     assert f.placement(h)[1] == "global"
 
 
+def case_lds_granules(f: Fake):
+    """LDS comes in granules of 1280 bytes: 32,396 a route (f32, dim 3072, Q =
+    256, full table) are 26 of 128, four routes a CU and not the five that
+    the bytes allow."""
+    h = f.context()
+    assert f.exact(h, f.L.ELEM_F32, 3072, 256, 4 * 256) == f.L.OK
+    assert f.placement(h)[1] == "lds"
+    assert f.exact(h, f.L.ELEM_F32, 3072, 256, 4 * 256 + 1) == f.L.OK
+    assert f.placement(h)[1] != "lds"
+
+
 def case_u8_slabs(f: Fake):
-    """u8 rows, 24 a CU with the spilling table and 28 with the slab: the
+    """u8 rows, 25 a CU with the spilling table and 28 with the slab: the
     slab up to a round (Q <= 72) or two of residents, or where a step reads
     less than 8 KB of rows."""
     f.hip.fake_waves(28)
@@ -195,11 +206,11 @@ def case_u8_slabs(f: Fake):
             h, p, L.ELEM_U8, dim, 1000, p, f.graph(degree), None, L.PredicateView(),
             f.routes(count), L.ExactParams(beam, 1, 2, 0, 10, 0), p, p, None) == L.OK
         return f.placement(h)[1]
-    # (the rows' LDS pads the spilling table to 24 a CU)
+    # (the rows' LDS pads the spilling table to 25 a CU)
     for dim, degree, beam, count, want in (
-            (1344, 8, 72, round_, "global"), (1344, 8, 72, round_ + 1, "spill"),
-            (1344, 8, 73, 2 * round_, "global"), (1344, 8, 73, 2 * round_ + 1, "spill"),
-            (1344, 6, 73, 2 * round_ + 1, "global"), (1344, 6, 72, round_ + 1, "spill"),
+            (1088, 8, 72, round_, "global"), (1088, 8, 72, round_ + 1, "spill"),
+            (1088, 8, 73, 2 * round_, "global"), (1088, 8, 73, 2 * round_ + 1, "spill"),
+            (1088, 6, 73, 2 * round_ + 1, "global"), (1088, 6, 72, round_ + 1, "spill"),
             (192, 64, 300, 60_000, "global")):
         assert placed(dim, degree, beam, count) == want, (dim, degree, beam, count)
 
