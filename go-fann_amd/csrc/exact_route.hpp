@@ -656,8 +656,22 @@ __global__ __launch_bounds__(64, (kElem == GOFANN_ELEM_U8 ? GOFANN_EXACT_MIN_WAV
     exact_route<kVisited, kC, kElem, 0>(a, lds);
 }
 
+// Waves per SIMD a set kernel is compiled for.  With four, two of its kinds
+// ran out of registers: f16 with the full LDS table spilled 16 at R = 2 (with
+// two waves' registers it takes 133, and the table leaves at most nine routes a
+// CU anyway; dim 512, Q = 64, 280 routes: 1.28 -> 1.22 ms), and long f32 rows at
+// R = 8 were scheduled into 95, the query read from LDS word by word between
+// the sums (with three waves' registers the reads go out ahead in 126, still
+// four waves; 2.7M rows of 16 KB, 6,666 routes at Q = 256 and 352: 187 -> 168 ms).
+template <int kVisited, int kC, int kElem>
+constexpr int set_min_waves()
+{
+    if (kElem == GOFANN_ELEM_F16 && kVisited == kVisitedLds) return 2;
+    return kElem == GOFANN_ELEM_F32 && kC < 0 ? 3 : 4;
+}
+
 template <int kVisited, int kC, int kElem, int kR>
-__global__ __launch_bounds__(64, 4) void exact_set_kernel(ExactArgs a)
+__global__ __launch_bounds__(64, (set_min_waves<kVisited, kC, kElem>())) void exact_set_kernel(ExactArgs a)
 {
     extern __shared__ __align__(16) unsigned char lds[];
     exact_route<kVisited, kC, kElem, kR>(a, lds);

@@ -45,7 +45,8 @@ def _resources(src: str, out_dir: Path) -> dict:
             continue
         for key, pat in (("vgprs", r"remark:\s+VGPRs: (\d+)"),
                          ("occupancy", r"remark:\s+Occupancy \[waves/SIMD\]: (\d+)"),
-                         ("vgpr_spill", r"remark:\s+VGPRs Spill: (\d+)")):
+                         ("vgpr_spill", r"remark:\s+VGPRs Spill: (\d+)"),
+                         ("scratch", r"remark:\s+ScratchSize \[bytes/lane\]: (\d+)")):
             m = re.search(pat, line)
             if m:
                 cur[key] = int(m.group(1))
@@ -55,7 +56,8 @@ def _resources(src: str, out_dir: Path) -> dict:
 @pytest.fixture(scope="module")
 def report(tmp_path_factory):
     d = tmp_path_factory.mktemp("res")
-    srcs = ("exact_route.hip", "pq_search_m48.hip", "pq_search_m32.hip", "rabitq_search.hip")
+    srcs = ("exact_route.hip", "exact_set_f16.hip", "exact_set_f32.hip", "exact_set_u8.hip",
+            "pq_search_m48.hip", "pq_search_m32.hip", "rabitq_search.hip")
     with ThreadPoolExecutor(max_workers=len(srcs)) as ex:
         return dict(zip(srcs, ex.map(lambda s: _resources(s, d), srcs)))
 
@@ -82,6 +84,21 @@ def test_exact_route_six_waves_without_step_spills(report):
         else:
             assert r["occupancy"] >= 4, (name, r)
             assert r["vgpr_spill"] == 0, (name, r)
+
+
+@pytest.mark.parametrize("elem", ["u8", "f16", "f32"])
+def test_exact_set_kernels_without_spills(report, elem):
+    """The set-frontier kernels, which float launches of beams up to 496 run:
+    no spill and no scratch memory, four waves a SIMD (three where the full
+    LDS table, first template argument 1, leaves at most nine routes a CU);
+    long f32 rows with more than 100 registers, which their 32 row words and
+    32 query words in flight need."""
+    for name, r in _kernels(report[f"exact_set_{elem}.hip"], "exact_set_kernel").items():
+        visited, long_rows = re.search(r"ILi(\d)EL(?:i0|in(1))E", name).groups()
+        assert r["vgpr_spill"] == 0 and r["scratch"] == 0, (name, r)
+        assert r["occupancy"] >= (3 if visited == "1" else 4), (name, r)
+        if elem == "f32" and long_rows:
+            assert r["vgprs"] > 100, (name, r)
 
 
 @pytest.mark.parametrize("src,needle", [
