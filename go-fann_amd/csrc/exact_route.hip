@@ -136,6 +136,7 @@ int launch_set_r(const LaunchShape& s, int chunks)
 template <int kElem>
 int launch_set(const LaunchShape& s, int chunks, int regs)
 {
+    if constexpr (kElem == GOFANN_ELEM_U8) return launch_set_r<kElem, 2>(s, chunks);
     switch (regs) {
     case 2: return launch_set_r<kElem, 2>(s, chunks);
     case 4: return launch_set_r<kElem, 4>(s, chunks);
@@ -205,13 +206,16 @@ static int exact_search_impl(Context* ctx, const void* base, int base_elem, uint
     const int fchunks = static_cast<size_t>(dim) * elem_bytes(base_elem) > kQuadMaxRowBytes ? -1 : 0;
     const uint32_t q = static_cast<uint32_t>(p->queue_limit);
     // The set frontier serves float rows, whose distances are seldom equal
-    // (4,900 f16 routes, dim 512: 9.9 ms, 10.5 with the heap), and u8
-    // launches of at most 16 routes: a u8 route without equal
-    // keys that matter runs in two thirds of the heap's time (248 against 369
-    // us), but one that has them replays its admissions on the heap, so the
-    // slowest of many is slower than with the heap (280 routes 1.16 against
-    // 1.04 ms), and a full chip's average is no better.
-    const bool set_pays = base_elem != GOFANN_ELEM_U8 || r->count <= 16;
+    // (4,900 f16 routes, dim 512: 9.9 ms, 10.5 with the heap), and u8 launches of
+    // at most 16 routes and beams of at most two registers a lane (Q = 112).  A
+    // u8 route that has equal keys which matter replays its admissions on the
+    // heap, so the wider the beam and the more routes, the likelier is one that
+    // takes longer than with the heap.  Set / heap, ms a launch at 1, 4, 16 and 32
+    // routes: dim 192, degree 64, Q = 32: 0.25 / 0.35, 0.30 / 0.41, 0.34 / 0.46,
+    // 0.37 / 0.48; Q = 112: 0.74 / 0.85, 0.89 / 0.94, 1.01 / 1.05, 1.10 / 1.10; Q =
+    // 128: 0.88 / 0.94, 1.06 / 1.03, 1.23 / 1.16, 1.33 / 1.21; dim 32, degree 32,
+    // Q = 72: 0.40 / 0.48, 0.51 / 0.55, 0.56 / 0.57, 0.65 / 0.59.
+    const bool set_pays = base_elem != GOFANN_ELEM_U8 || (r->count <= 16 && q + kSetSlack <= 128);
     if (const int regs = fixed_slab == nullptr && set_pays
                              ? set_registers(ctx, p->queue_limit, r->count, &a.log) : 0) {
         a.log_mask = set_log_entries(p->queue_limit) - 1u;

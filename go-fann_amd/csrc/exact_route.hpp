@@ -796,7 +796,7 @@ int launch_exact(Context* ctx, ExactArgs& a, int hash_mode, uint32_t lds_full,
     prefix template int launch_exact<-1, elem, 2>(GOFANN_EXACT_LAUNCH_ARGS);            \
     prefix template int launch_exact<-1, elem, 4>(GOFANN_EXACT_LAUNCH_ARGS);            \
     prefix template int launch_exact<-1, elem, 8>(GOFANN_EXACT_LAUNCH_ARGS);
-GOFANN_EXACT_SET_LAUNCHES(extern, GOFANN_ELEM_U8)
+extern template int launch_exact<0, GOFANN_ELEM_U8, 2>(GOFANN_EXACT_LAUNCH_ARGS);
 GOFANN_EXACT_SET_LAUNCHES(extern, GOFANN_ELEM_F32)
 GOFANN_EXACT_SET_LONG_LAUNCHES(extern, GOFANN_ELEM_F32)
 GOFANN_EXACT_SET_LAUNCHES(extern, GOFANN_ELEM_F16)

@@ -4,6 +4,6 @@
 
 namespace gofann {
 
-GOFANN_EXACT_SET_LAUNCHES(, GOFANN_ELEM_U8)
+template int launch_exact<0, GOFANN_ELEM_U8, 2>(GOFANN_EXACT_LAUNCH_ARGS);
 
 }  // namespace gofann

@@ -354,8 +354,8 @@ def test_exact_search_rejects_bad_params(gpu_ctx, eworld):
         assert rc in (_lib.ERR_INVALID, _lib.ERR_UNSUPPORTED)
 
 
-# ---- the set frontier (set_frontier.hpp), which launches of at most 16
-# routes take
+# ---- the set frontier (set_frontier.hpp), which float launches take, and u8
+# launches of at most 16 routes and beams up to 112
 def _sixteens(rs):
     """The routes sixteen at a time, then the heap's seventeen."""
     for a, b in [(a, min(rs.count, a + 16)) for a in range(0, rs.count, 16)] + [(0, 17)]:
@@ -368,10 +368,9 @@ def _sixteens(rs):
 @pytest.mark.parametrize("shift", [4, 6, 7])
 @pytest.mark.parametrize("Q", [2, 7, 48, 111, 112, 113, 240, 241, 496, 497])
 def test_exact_search_equal_distances(gpu_ctx, eworld, shift, Q):
-    """Beams around every register count of the set frontier (112, 240 and
-    496 are the last of two, four and eight; 497 takes the heap) over rows
-    of 16, 4 and 2 distinct values a dim: many equal distances, so that the
-    order of the heap decides who is next and who leaves."""
+    """Rows of 16, 4 and 2 distinct values a dim: many equal distances, so
+    that the order of the heap decides who is next and who leaves.  The set
+    frontier serves the u8 beams up to 112, the heap those past it."""
     wl, li, rs = eworld
     say("exact search, equal distances", shift, "Q", Q)
     rows = (wl.base.numpy()[:, :12] >> shift, wl.queries.numpy()[:, :12] >> shift)
@@ -383,6 +382,25 @@ def test_exact_search_equal_distances(gpu_ctx, eworld, shift, Q):
     for part in _sixteens(rs):
         _run(gpu_ctx, Small, li, part, None, lambda dr, dg: _lib.PredicateView(), Q, 10, 2,
              _lib.PLACE_AUTO, False, rows=rows)
+
+
+@pytest.mark.parametrize("Q", [2, 111, 112, 113, 240, 241, 496, 497])
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+def test_exact_search_equal_float_distances(gpu_ctx, eworld, dtype, Q):
+    """The same for float rows, which take the set frontier whatever the
+    number of routes: integer rows of 4 distinct values a dim (their sums are
+    exact in either type).  112, 240 and 496 are the last beams of two, four
+    and eight registers a lane; 497 takes the heap."""
+    wl, li, rs = eworld
+    say("exact search, equal float distances", dtype, "Q", Q)
+    dt = np.float32 if dtype == "f32" else np.float16
+    rows = tuple(np.ascontiguousarray((r.numpy()[:, :12] >> 6).astype(dt))
+                 for r in (wl.base, wl.queries))
+
+    class Small:
+        dim, n = 12, wl.n
+    _run(gpu_ctx, Small, li, rs, None, lambda dr, dg: _lib.PredicateView(), Q, 10, 2,
+         _lib.PLACE_AUTO, False, rows=rows)
 
 
 def _run_both(ctx, li, rs, base, q, Q, mode):
@@ -439,11 +457,10 @@ def test_exact_search_unordered_distances(gpu_ctx, eworld, dtype, Q, kind):
             assert np.array_equal(x, y)
 
 
-def test_exact_search_log_ring_wraps(gpu_ctx, eworld):
-    """Routes without early stop admit more entries than the log ring of a
-    small beam holds (1024), so that the ring brings the heap up to date."""
+def test_exact_search_without_early_stop(gpu_ctx, eworld):
+    """Whole routes: the set frontier gives what the heap frontier gives."""
     wl, li, rs = eworld
-    say("exact search, log ring")
+    say("exact search, no early stop")
     rng = np.random.default_rng(3)
     base = rng.standard_normal((wl.n, 32)).astype(np.float32)
     q = rng.standard_normal((wl.queries.shape[0], 32)).astype(np.float32)
@@ -452,6 +469,41 @@ def test_exact_search_log_ring_wraps(gpu_ctx, eworld):
             a, b = _run_both(gpu_ctx, li, part, base, q, Q, 1)
             for x, y in zip(a, b):
                 assert np.array_equal(x, y)
+
+
+def _line_world(n, degree=32):
+    """One group whose row i links to the next `degree` rows, each nearer to
+    the queries than the last, the seed farthest: a search admits every row.
+    The last 400 rows are four at each of 100 distances."""
+    i = np.arange(n, dtype=np.int64)
+    nxt = i[:, None] + 1 + np.arange(degree)[None, :]
+    graph = np.where(nxt < n, nxt, U32MAX).astype(np.uint32)
+    rows = i.astype(np.uint32)
+    li = gi.LabelIndex(1, 0, np.array([n]), np.zeros(1, np.uint32), np.array([n], np.uint32), rows,
+                       graph, np.zeros(1, np.uint32), np.array([0, n], np.uint64), rows,
+                       np.arange(n + 1, dtype=np.uint32), np.zeros(n, np.uint32), degree)
+    rs = gp._routeset([(q, 0, [], []) for q in range(6)], li)
+    x = np.zeros((n, 8), np.float32)
+    x[:, 0] = n - i
+    x[-400:, 0] = np.repeat(np.arange(100, 0, -1), 4)
+    q = np.zeros((6, 8), np.float32)
+    q[:, 1] = np.arange(6)
+    return li, rs, x, q
+
+
+@pytest.mark.parametrize("Q,ring", [(2, 1024), (112, 1024), (113, 2048), (496, 2048)])
+def test_exact_search_log_ring_wraps(gpu_ctx, Q, ring):
+    """Routes that admit more than twice what the log ring holds, with no
+    equal keys until the end: a full ring brings the heap up to date, and
+    the order among the equal keys that follow depends on all of it."""
+    say("exact search, log ring", Q)
+    li, rs, x, q = _line_world(6000)
+
+    class Line:
+        dim, n = 8, 6000
+    _, st = _run(gpu_ctx, Line, li, rs, None, lambda dr, dg: _lib.PredicateView(), Q, 10, 1,
+                 _lib.PLACE_AUTO, False, rows=(x, q))
+    assert st[:, 6].min() > 2 * ring
 
 
 def test_exact_scan_beside_a_capture(gpu_ctx, scan_worlds):

@@ -153,6 +153,20 @@ def case_captured_launches_keep_no_scratch(f: Fake):
     assert [g for _, g in f.launched()] == [128, 8]
 
 
+def case_u8_set_frontier(f: Fake):
+    """u8 rows take the set frontier up to 16 routes and Q = 112, float rows at
+    any number and up to Q = 496."""
+    h = f.context()
+    for elem, beam, count, regs in ((f.L.ELEM_U8, 112, 16, 2), (f.L.ELEM_U8, 113, 1, 0),
+                                    (f.L.ELEM_U8, 2, 17, 0), (f.L.ELEM_U8, 200, 16, 0),
+                                    (f.L.ELEM_F16, 112, 999, 2), (f.L.ELEM_F16, 113, 1, 4),
+                                    (f.L.ELEM_F32, 240, 17, 4), (f.L.ELEM_F32, 241, 17, 8),
+                                    (f.L.ELEM_F32, 496, 1, 8), (f.L.ELEM_F32, 497, 1, 0)):
+        assert f.exact(h, elem, 64, beam, count) == f.L.OK
+        [(name, _)] = f.launched()
+        assert exact_kernel(name)[1] == regs, (elem, beam, count)
+
+
 def case_full_table_beside_others(f: Fake):
     """The full LDS table: every resident launch on the default stream; up to
     a quarter of a CU's LDS on a stream that may run beside others."""
