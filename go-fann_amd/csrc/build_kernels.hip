@@ -2015,14 +2015,16 @@ template <class T>
 int bucket_reps_t(Context* ctx, const T* rows, uint32_t dim, const uint32_t* bucket_offsets,
                   uint32_t buckets, uint32_t n, float* means, uint32_t* reps)
 {
-    if (!row_vectors(rows, static_cast<size_t>(dim) * sizeof(T)) ||
-        (reinterpret_cast<uintptr_t>(means) & 15u) != 0) {
+    // one workgroup per bucket also where there is no memory for the keys
+    unsigned long long* keys = nullptr;
+    if (row_vectors(rows, static_cast<size_t>(dim) * sizeof(T)) &&
+        (reinterpret_cast<uintptr_t>(means) & 15u) == 0)
+        keys = static_cast<unsigned long long*>(
+            ctx->optional_scratch(Context::kScratchBuild, static_cast<size_t>(buckets) * 8));
+    if (keys == nullptr) {
         hipLaunchKernelGGL(bucket_rep_kernel<T>, dim3(buckets), dim3(kThreads), 0, ctx->stream, rows, dim,
                            bucket_offsets, means, reps);
     } else {
-        unsigned long long* keys = static_cast<unsigned long long*>(
-            ctx->scratch(Context::kScratchBuild, static_cast<size_t>(buckets) * 8));
-        if (!keys) return ctx->fail(GOFANN_ERR_NOMEM, "bucket representative scratch allocation failed");
         constexpr int kV = 4 / static_cast<int>(sizeof(T));
         hipLaunchKernelGGL((bucket_mean_kernel<T, kV>), dim3(buckets, (dim + kWave * kV - 1) / (kWave * kV)),
                            dim3(kWave), 0, ctx->stream, rows, dim, bucket_offsets, means, keys);

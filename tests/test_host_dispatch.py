@@ -153,6 +153,21 @@ def case_captured_launches_keep_no_scratch(f: Fake):
     assert [g for _, g in f.launched()] == [128, 8]
 
 
+def case_bucket_reps_without_memory(f: Fake):
+    """Bucket representatives need no buffer: without memory for the keys, one
+    workgroup per bucket."""
+    h = f.context()
+    off = (C.c_uint32 * 5)(0, 8, 16, 24, 32)
+    for limit, kernels in ((0, ["bucket_rep_kernel"]),
+                           (GIB, ["bucket_mean_kernel", "bucket_dist_kernel",
+                                  "bucket_pick_kernel"])):
+        f.hip.fake_limit(f.hip.fake_used() + limit)
+        assert f.lib.gofann_build_bucket_reps(h, f.p, f.L.ELEM_F32, 64, C.addressof(off), 4, f.p,
+                                              f.p) == f.L.OK
+        names = [n for n, _ in f.launched()]
+        assert len(names) == len(kernels) and all(k in n for k, n in zip(kernels, names)), names
+
+
 def case_u8_set_frontier(f: Fake):
     """u8 rows take the set frontier up to 16 routes and Q = 112, float rows at
     any number and up to Q = 496."""
