@@ -1698,6 +1698,9 @@ int knn_t(Context* ctx, const T* rows, uint32_t dim, const gofann_build_buckets*
     // without a tile (256 centres of 512 dims, k = 4, is 4 tiles of 64:
     // 459 us, as 16 of 16 rows 113 us).
     const int kq = whole < static_cast<uint64_t>(ctx->compute_units) ? 16 : kTile;
+    const size_t lds = (kKnnStage + static_cast<size_t>(kq) * k * 2) * 4;
+    if (lds > static_cast<size_t>(ctx->lds_per_block))
+        return ctx->fail(GOFANN_ERR_UNSUPPORTED, "kNN list exceeds the workgroup LDS");
     std::vector<uint32_t> list;  // bucket of every tile, then first row of every tile
     for (uint32_t i : by)
         for (uint64_t r = off[i]; r < off[i + 1]; r += kq) list.push_back(i);
@@ -1709,9 +1712,6 @@ int knn_t(Context* ctx, const T* rows, uint32_t dim, const gofann_build_buckets*
     if (!dev) return ctx->fail(GOFANN_ERR_NOMEM, "kNN scratch allocation failed");
     if (hipMemcpyAsync(dev, list.data(), list.size() * 4, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
         return ctx->fail_hip("kNN tile list copy");
-    const size_t lds = (kKnnStage + static_cast<size_t>(kq) * k * 2) * 4;
-    if (lds > static_cast<size_t>(ctx->lds_per_block))
-        return ctx->fail(GOFANN_ERR_UNSUPPORTED, "kNN list exceeds the workgroup LDS");
     const auto launch = [&](auto kern) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
