@@ -312,3 +312,26 @@ def test_knn_many_tiles_match_oracle(hip, dtype, dim):
     want, _ = po.build_knn(x, off, 16)
     got = hip.knn(hip.rows(torch.from_numpy(x)), off, 16)
     assert np.array_equal(_u32(got), want)
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("dim", [24, 33])
+def test_knn_many_tiles_probe_lists_match_oracle(hip, dtype, dim):
+    """64-row query tiles that scan the buckets of a probe list: empty
+    buckets on the lists, lists of one and of many, some without their own
+    bucket (of which one is empty)."""
+    say("knn tiles with probe lists", dtype.__name__, dim)
+    rng = np.random.default_rng(dim * 5 + 2)
+    sizes = np.concatenate([rng.integers(1, 30, size=270), [300, 129, 0, 64, 65]])
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint32)
+    nb = len(sizes)
+    lists = [rng.permutation(nb)[: int(m)] for m in rng.integers(1, 6, size=nb)]
+    for b in range(0, nb, 2):
+        lists[b] = np.concatenate([[b], lists[b][lists[b] != b]])
+    lists[3], lists[nb - 5] = np.array([nb - 3, 1, nb - 5]), np.arange(nb)
+    poff = np.concatenate([[0], np.cumsum([len(l) for l in lists])]).astype(np.uint32)
+    probe = np.concatenate(lists).astype(np.uint32)
+    x = _rows(rng, int(off[-1]), dim, dtype)
+    want, _ = po.build_knn(x, off, 16, poff, probe)
+    got = hip.knn(hip.rows(torch.from_numpy(x)), off, 16, poff, probe)
+    assert np.array_equal(_u32(got), want)

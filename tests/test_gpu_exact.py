@@ -543,3 +543,58 @@ def test_exact_scan_beside_a_capture(gpu_ctx, scan_worlds):
     assert np.array_equal(out[1].cpu().numpy().reshape(n, 10).view(np.uint32),
                           want[1].view(np.uint32))
     ctx.close()
+
+
+def test_exact_searches_beside_a_scan(gpu_ctx, eworld, scan_worlds):
+    """Two contexts on streams of their own, searches on one beside scans on
+    the other, alternating batch sizes: each gives what it gives alone."""
+    wl, li, rs = eworld
+    say("exact searches beside a scan")
+    dg, dr = gs.DeviceGraph.upload(li), gs.DeviceRoutes.upload(rs)
+    base, q = wl.base.float().cuda(), wl.queries.float().cuda()
+    ls = gs.u32(li.label_size)
+    n = int(q.shape[0])
+    rng = np.random.default_rng(12)
+    ids = rng.integers(0, wl.n, n * 900).astype(np.uint32)
+    lists = [gs.u32(a) for a in (np.arange(n, dtype=np.uint32), ids,
+                                 np.arange(n, dtype=np.uint32) * 900, np.full(n, 900, np.uint32))]
+
+    def search(ctx, count, out):
+        prm = _lib.ExactParams(96, 1, 2, 0, 10, _lib.PLACE_AUTO)
+        ctx.check(ctx.lib.gofann_exact_search(
+            ctx.handle, _lib.ptr(base), _lib.ELEM_F32, wl.dim, wl.n, _lib.ptr(q), dg.view(),
+            _lib.ptr(ls), _lib.PredicateView(), dr.routes_view(0, count), prm, _lib.ptr(out[0]),
+            _lib.ptr(out[1]), None))
+
+    def scan(ctx, count, out):
+        ctx.check(ctx.lib.gofann_exact_posting_scan(
+            ctx.handle, _lib.ptr(base), _lib.ELEM_F32, wl.dim, wl.n, _lib.ptr(q),
+            _lib.PredicateView(), *[_lib.ptr(t) for t in lists], count, 10,
+            _lib.EXACT_ORDER_SERIAL, _lib.ptr(out[0]), _lib.ptr(out[1]), None))
+
+    def buffers():
+        return (torch.zeros(max(n, rs.count) * 10, dtype=torch.int32, device="cuda"),
+                torch.zeros(max(n, rs.count) * 10, device="cuda"))
+
+    counts = [(3, n), (rs.count, 5), (17, n), (rs.count, n)]
+    want = []
+    for a, b in counts:
+        o = buffers(), buffers()
+        search(gpu_ctx, a, o[0])
+        scan(gpu_ctx, b, o[1])
+        want.append(o)
+    ctxs, streams = [_lib.Context(0) for _ in range(2)], [torch.cuda.Stream() for _ in range(2)]
+    got = [(buffers(), buffers()) for _ in counts]
+    torch.cuda.synchronize()
+    for c, s in zip(ctxs, streams):
+        c.bind_stream(s)
+    for (a, b), o in zip(counts, got):
+        search(ctxs[0], a, o[0])
+        scan(ctxs[1], b, o[1])
+    torch.cuda.synchronize()
+    for w, g in zip(want, got):
+        for x, y in zip(w, g):
+            assert torch.equal(x[0], y[0])
+            assert torch.equal(x[1].view(torch.int32), y[1].view(torch.int32))
+    for c in ctxs:
+        c.close()
