@@ -1102,6 +1102,7 @@ struct Placement {
     int visited;  // kVisitedGlobal / kVisitedLds / kVisitedSpill
     uint32_t lds;
     int resident;
+    int most;     // residents of the placement that holds the most, of those allowed
 };
 
 // Visited-set placement for one scorer configuration.  hash_mode picks it;
@@ -1112,23 +1113,22 @@ struct Placement {
 template <class Scorer>
 Placement choose_visited(Context* ctx, const Layout& l, int hash_mode, uint32_t routes)
 {
-    const Placement full{kVisitedLds, l.bytes(kVisitedLds),
-                         resident_per_cu(ctx, traversal_kernel<Scorer, kVisitedLds>,
-                                         l.bytes(kVisitedLds))};
-    const Placement spill{kVisitedSpill, l.bytes(kVisitedSpill),
-                          resident_per_cu(ctx, traversal_kernel<Scorer, kVisitedSpill>,
-                                          l.bytes(kVisitedSpill))};
-    const Placement glob{kVisitedGlobal, l.bytes(kVisitedGlobal),
-                         resident_per_cu(ctx, traversal_kernel<Scorer, kVisitedGlobal>,
-                                         l.bytes(kVisitedGlobal))};
+    const auto at = [&](int visited, auto kern) {
+        const int r = resident_per_cu(ctx, kern, l.bytes(visited));
+        return Placement{visited, l.bytes(visited), r, r};
+    };
+    Placement full = at(kVisitedLds, traversal_kernel<Scorer, kVisitedLds>);
+    const Placement spill = at(kVisitedSpill, traversal_kernel<Scorer, kVisitedSpill>);
+    const Placement glob = at(kVisitedGlobal, traversal_kernel<Scorer, kVisitedGlobal>);
     if (hash_mode == GOFANN_PLACE_LDS) return full;
     if (hash_mode == GOFANN_PLACE_GLOBAL) return glob;
     if (hash_mode == GOFANN_PLACE_SPILL) return spill;
-    if (full_table(ctx, routes, full.lds, full.resident)) return full;
     Placement best = full;
     if (spill.resident > best.resident) best = spill;
     if (glob.resident > best.resident) best = glob;
-    return best;
+    if (!full_table(ctx, routes, full.lds, full.resident)) return best;
+    full.most = best.most;
+    return full;
 }
 
 template <class Scorer>
@@ -1195,8 +1195,9 @@ PqScorer<kM, kSub> make_pq_scorer(const gofann_pq_view* pq, const void* queries,
     return sc;
 }
 
-// PQ: choose the table placement (LDS table vs on-demand entries) and the
-// visited-set placement by resident routes per CU, then launch.
+// PQ: choose the table placement (LDS table vs on-demand entries) by the most
+// routes per CU that each form can hold, whatever visited placement its launch
+// takes (a launch small enough for the full table holds fewer), then launch.
 template <int kM, int kMD, int kSub>
 int pq_search_ms(Context* ctx, const gofann_pq_view* pq, const void* queries, int query_elem,
                  const gofann_graph_view* g, const gofann_predicate_view* pred,
@@ -1209,11 +1210,11 @@ int pq_search_ms(Context* ctx, const gofann_pq_view* pq, const void* queries, in
                                   p->result_width);
     const Layout ld = make_layout(DirectScorer::lds_bytes(pq->dim, pq->pq_dim), p->queue_limit,
                                   p->result_width);
-    Placement pt{kVisitedGlobal, 0, 0}, pd{kVisitedGlobal, 0, 0};
+    Placement pt{kVisitedGlobal, 0, 0, 0}, pd{kVisitedGlobal, 0, 0, 0};
     if (p->table_mode != GOFANN_PLACE_GLOBAL) pt = choose_visited<TableScorer>(ctx, lt, p->hash_mode, r->count);
     if (p->table_mode != GOFANN_PLACE_LDS) pd = choose_visited<DirectScorer>(ctx, ld, p->hash_mode, r->count);
     const bool direct = p->table_mode == GOFANN_PLACE_GLOBAL ||
-                        (p->table_mode == GOFANN_PLACE_AUTO && pd.resident > pt.resident);
+                        (p->table_mode == GOFANN_PLACE_AUTO && pd.most > pt.most);
     ctx->last_table_in_lds = direct ? 0 : 1;
     if (direct)
         return launch_traversal(ctx, make_pq_scorer<kMD, kSub>(pq, queries, query_elem), ld, pd, g,

@@ -81,6 +81,13 @@ class Fake:
                                              self.graph(), L.PredicateView(), self.routes(count),
                                              prm, p, p, None)
 
+    def pq(self, ctx, m, beam, count):
+        L, p = self.L, self.p
+        prm = L.SearchParams(beam, 1, 2, 0, 10, 100, 0.0, 0.0, 0, 0, 0, 0)
+        return self.lib.gofann_pq_search(ctx, L.PqView(p, p, 4 * m, m, 1000, None, 0), p,
+                                         L.ELEM_F32, self.graph(), L.PredicateView(),
+                                         self.routes(count), prm, p, p, None)
+
     def placement(self, ctx):
         """(PQ table in LDS, visited placement) of the last launch."""
         v = [C.c_int() for _ in range(4)]
@@ -196,6 +203,17 @@ def case_full_table_beside_others(f: Fake):
         assert f.rabitq(h, 4096, 320, per_cu * 256) == f.L.OK
         want = "lds" if stream == 0 or per_cu == 1 else "global"
         assert f.placement(h)[1] == want, (stream, per_cu)
+
+
+def case_pq_form(f: Fake):
+    """PQ's form (table in LDS or entries on demand) does not depend on the
+    visited placement that a launch of the size takes: with 16 subspaces the
+    entries on demand hold twice the routes of the table (16 a CU, 8), also
+    where their full table holds only 8."""
+    for count in (1, 1000, 1800, 2048, 2049, 9000):
+        h = f.context()
+        assert f.pq(h, 16, 64, count) == f.L.OK
+        assert f.placement(h) == (0, "lds" if count <= 2048 else "spill"), count
 
 
 def case_most_residents(f: Fake):
