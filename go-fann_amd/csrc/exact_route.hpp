@@ -694,10 +694,12 @@ int exact_resident(Context* ctx, uint32_t lds)
 }
 
 // Whether the visited slabs' memory traffic (16 KB a route) is felt: u8
-// launches of more than one round of resident routes whose sets mostly stay
-// within the spilling table (Q <= 72), and of more than two rounds where
-// the rows' own traffic is high (degree x dim of 8 KB a step or more).  The
-// spilling table (23-24 routes a CU) against the slab (28), ms at dim x degree:
+// launches whose sets mostly stay within the spilling table (Q <= 64; at Q <= 72
+// those of more than one round of resident routes), and of more than two
+// rounds where the rows' own traffic is high (degree x dim of 8 KB a step or
+// more).  The spilling table (23-24 routes a CU) against the slab (28), ms at
+// dim x degree:
+//   192 x 64, Q = 32: 3,000 routes 0.89 / 0.92, 12,000 1.52 / 1.76
 //   192 x 64, Q = 72: 5,000 routes 2.07 / 1.99, 20,000 5.02 / 5.68, 57,000
 //     11.7 / 14.2; Q = 96: 2.53 / 2.43, 6.77 / 7.13, 16.5 / 17.8; 12,000 at
 //     Q = 112 4.36 / 4.07
@@ -712,7 +714,7 @@ bool slabs_cost(const Context* ctx, const ExactArgs& a, uint32_t count, int resi
 {
     if (kElem != GOFANN_ELEM_U8) return false;
     const uint64_t round = static_cast<uint64_t>(residents) * static_cast<uint64_t>(ctx->compute_units);
-    if (a.params.queue_limit <= 72) return count > round;
+    if (a.params.queue_limit <= 72) return a.params.queue_limit <= 64 || count > round;
     return count > 2 * round && static_cast<uint64_t>(a.dim) * a.graph.degree >= 8192;
 }
 

@@ -216,6 +216,17 @@ def case_pq_form(f: Fake):
         assert f.placement(h) == (0, "lds" if count <= 2048 else "spill"), count
 
 
+def case_narrow_beams_spill(f: Fake):
+    """A narrow beam's launch that the spilling table holds (21 routes a CU)
+    takes it, though the slab would hold more (28)."""
+    f.hip.fake_waves(28)
+    h = f.context()
+    for beam, count, want in ((80, 21 * 256, "spill"), (81, 21 * 256, "global"),
+                              (80, 21 * 256 + 1, "global")):
+        assert f.pq(h, 32, beam, count) == f.L.OK
+        assert f.placement(h)[1] == want, (beam, count)
+
+
 def case_most_residents(f: Fake):
     """Past the full table, the most resident routes a CU, also where the
     spilling table holds the whole launch."""
@@ -242,8 +253,8 @@ def case_lds_granules(f: Fake):
 
 def case_u8_slabs(f: Fake):
     """u8 rows, 25 a CU with the spilling table and 28 with the slab: the
-    slab up to a round (Q <= 72) or two of residents, or where a step reads
-    less than 8 KB of rows."""
+    spilling table at Q <= 64, past a round of residents at Q <= 72, past two
+    where a step reads 8 KB of rows."""
     f.hip.fake_waves(28)
     h, round_ = f.context(), 28 * 256
 
@@ -255,6 +266,7 @@ def case_u8_slabs(f: Fake):
         return f.placement(h)[1]
     # (the rows' LDS pads the spilling table to 25 a CU)
     for dim, degree, beam, count, want in (
+            (1088, 4, 64, 5000, "spill"), (1088, 8, 65, 5000, "global"),
             (1088, 8, 72, round_, "global"), (1088, 8, 72, round_ + 1, "spill"),
             (1088, 8, 73, 2 * round_, "global"), (1088, 8, 73, 2 * round_ + 1, "spill"),
             (1088, 6, 73, 2 * round_ + 1, "global"), (1088, 6, 72, round_ + 1, "spill"),
