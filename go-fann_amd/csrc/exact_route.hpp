@@ -697,12 +697,12 @@ int exact_resident(Context* ctx, uint32_t lds)
 // launches whose sets mostly stay within the spilling table (Q <= 64; at Q <= 72
 // those of more than one round of resident routes), and of more than two
 // rounds where the rows' own traffic is high (degree x dim of 8 KB a step or
-// more).  The spilling table (23-24 routes a CU) against the slab (28), ms at
-// dim x degree:
+// more).  The spilling table (24 routes a CU up to Q = 80, 21 to Q = 128) against
+// the slab (28), ms at dim x degree:
 //   192 x 64, Q = 32: 3,000 routes 0.89 / 0.92, 12,000 1.52 / 1.76
 //   192 x 64, Q = 72: 5,000 routes 2.07 / 1.99, 20,000 5.02 / 5.68, 57,000
 //     11.7 / 14.2; Q = 96: 2.53 / 2.43, 6.77 / 7.13, 16.5 / 17.8; 12,000 at
-//     Q = 112 4.36 / 4.07
+//     Q = 112 4.36 / 4.07; 57,000 at Q = 128 21.8 / 22.2
 //   96 x 32, Q = 64: 6,000 1.84 / 1.81, 45,000 8.13 / 8.34; Q = 96: 2.94 /
 //     2.38, 12.5 / 11.5
 //   96 x 64, Q = 96: 12,000 4.43 / 3.84, 45,000 12.1 / 12.1; 128 x 48: 45,000
@@ -721,7 +721,7 @@ bool slabs_cost(const Context* ctx, const ExactArgs& a, uint32_t count, int resi
 // Visited-set placement, then the launch.  Auto: the full LDS table where
 // full_table says so, else the most resident routes per CU, LDS preferred on
 // ties; where the slabs' traffic costs more than residents gain
-// (slabs_cost), the global slab has to hold a quarter more of them.
+// (slabs_cost), the global slab has to hold more than a third more of them.
 // fixed_slab: visited slabs for a placement outside LDS, holding at most
 // fixed_routes routes (the no-alloc entry point); nullptr: context scratch.
 template <int kC, int kElem, int kR>
@@ -746,7 +746,7 @@ int launch_exact(Context* ctx, ExactArgs& a, int hash_mode, uint32_t lds_full,
                 mode = kVisitedSpill;
                 res = rs;
             }
-            if (rg > res + (slabs_cost<kElem>(ctx, a, count, rg) ? res / 4 : 0)) {
+            if (rg > res + (slabs_cost<kElem>(ctx, a, count, rg) ? res / 3 : 0)) {
                 mode = kVisitedGlobal;
                 res = rg;
             }

@@ -179,8 +179,8 @@ typedef struct {
      * it, on a stream other than the default one only up to a quarter of the
      * LDS; other launches take the placement with the most resident routes per
      * CU (narrow PQ and RaBitQ beams: the spilling table where it holds the
-     * whole launch; exact route, large u8 launches: the slab only if it holds a
-     * quarter more than the spilling table). */
+     * whole launch; exact route, large u8 launches: the slab only if it holds
+     * over a third more than the spilling table). */
     int table_mode;
     int hash_mode;
 } gofann_search_params;

@@ -270,6 +270,8 @@ def case_u8_slabs(f: Fake):
             (1088, 8, 72, round_, "global"), (1088, 8, 72, round_ + 1, "spill"),
             (1088, 8, 73, 2 * round_, "global"), (1088, 8, 73, 2 * round_ + 1, "spill"),
             (1088, 6, 73, 2 * round_ + 1, "global"), (1088, 6, 72, round_ + 1, "spill"),
+            (1088, 8, 100, 2 * round_ + 1, "spill"),    # 21 a CU: a third of it more
+            (1088, 8, 160, 2 * round_ + 1, "global"),   # 18 a CU
             (192, 64, 300, 60_000, "global")):
         assert placed(dim, degree, beam, count) == want, (dim, degree, beam, count)
 
