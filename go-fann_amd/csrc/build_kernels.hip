@@ -499,8 +499,9 @@ __global__ __launch_bounds__(kThreads) void kpp_min_kernel(const T* rows, uint32
 // floor(u * n) when every distance is zero).  Writes the pick and copies
 // its row to centre j.  32,768 x 512 f16 rows, 256 centres: with the chunk sums
 // and a second serial pass in this one workgroup a pick took 45.8 us, now
-// 17.2 (most of it the chain of 1024 adds); the distance update 15.3, now 10.1
-// with four rows of a wave in flight and the chunk sums included.
+// 17.2, about 40 cycles for each of the 1024 sums that the one thread reads from
+// LDS, adds and writes back, if that loop is all of it; the distance update 15.3,
+// now 10.1 with four rows of a wave in flight and the chunk sums included.
 template <class T>
 __global__ __launch_bounds__(1024) void kpp_pick_kernel(const T* rows, uint32_t dim, uint64_t n,
                                                         uint64_t chunk, uint32_t nchunks,

@@ -30,7 +30,7 @@ constexpr int kExactMaxTopk = 10;  // defaults::max_topk
 // 6 holds them to 80 VGPRs, 24 routes per CU, without spills (the lane id and
 // the arguments are taken anew per step).  At C2, Q = 80: 46.1 ms, against 49.0
 // at 5 waves and 54.1 at 7 (the visited table leaves LDS).  The f32 / f16 kernels
-// (eight partial sums and two 16-byte loads per lane) take 5: at 6 they spill.
+// (eight partial sums and two 16-byte loads per lane) take fewer (below).
 #ifndef GOFANN_EXACT_MIN_WAVES
 #define GOFANN_EXACT_MIN_WAVES 6
 #endif
@@ -455,8 +455,9 @@ __device__ __forceinline__ void exact_route(const ExactArgs& args, unsigned char
         // per step: lane-derived values are not held across steps (no spills
         // at 6 waves; with the lane hoisted out of the loop, 10 VGPRs spilled),
         const int lane = opaque_lane(wave_lane);
-        // nor are the arguments (105-128 scalar registers spilled into vector
-        // lanes, 8-18 now)
+        // nor are the arguments (held over the route, 105-128 scalar registers
+        // were spilled into vector lanes; read per step, 6-21 in the heap's
+        // kernels and 19-53 in the set's)
         const ExactArgs& a = step_args<ExactArgs>();
         if (a.params.max_steps != 0 && steps >= static_cast<uint32_t>(a.params.max_steps)) break;
 

@@ -732,11 +732,11 @@ __global__ __launch_bounds__(64, GOFANN_TRAVERSAL_MIN_WAVES) void traversal_kern
     const int wave_lane = lane;
     while (step == 0 || heap_size > 1) {
         // per step: lane-derived values are not held across steps (PqScorer<48>
-        // 111 VGPRs, RaBitQ 118-120, no spills; with the lane hoisted out of
+        // 100-108 VGPRs, RaBitQ 116-120, no spills; with the lane hoisted out of
         // the loop both reach the 128-VGPR budget and spill)
         const int lane = opaque_lane(wave_lane);
         // and so are the arguments (step_args: 309-358 scalar registers of the
-        // RaBitQ kernels were spilled into vector lanes, 100-114 are)
+        // RaBitQ kernels were spilled into vector lanes, 100-116 are)
         constexpr uint32_t kScorerAt = (sizeof(TraversalArgs) + alignof(Scorer) - 1) / alignof(Scorer) *
                                        alignof(Scorer);
         const TraversalArgs& a = step_args<TraversalArgs>();
