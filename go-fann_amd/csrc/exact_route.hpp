@@ -694,12 +694,16 @@ int exact_resident(Context* ctx, uint32_t lds)
         ctx, reinterpret_cast<const void*>(exact_kernel<kVisited, kC, kElem, kR>()), lds);
 }
 
-// Whether the visited slabs' memory traffic (16 KB a route) is felt: u8
-// launches whose sets mostly stay within the spilling table (Q <= 64; at Q <= 72
-// those of more than one round of resident routes), and of more than two
-// rounds where the rows' own traffic is high (degree x dim of 8 KB a step or
-// more).  The spilling table (24 routes a CU up to Q = 80, 21 to Q = 128) against
-// the slab (28), ms at dim x degree:
+// Whether the spilling table pays where the slab holds up to a third more
+// routes.  u8 rows: narrow beams (at Q <= 72 also launches of more than one
+// round of resident routes), and launches of more than two rounds where the
+// rows' own traffic is high (degree x dim of 8 KB a step or more), which the
+// slabs' (16 KB a route) adds to.  The spilling table (24 routes a CU up to Q =
+// 80, 21 to Q = 128) against the slab (28), ms at dim x degree:
+//   89 x 64, 2,800 routes, 1,800 rows a group: Q = 64 0.71 / 0.86, Q = 111 1.12 /
+//     1.31, Q = 160 1.60 / 1.78, Q = 224 2.50 / 2.40; 7,400 rows: Q = 160 1.87 / 1.95,
+//     Q = 224 3.36 / 2.62; 14,800: Q = 111 1.61 / 1.64, Q = 160 2.36 / 2.20; 44,000:
+//     Q = 64 1.36 / 1.41, Q = 111 2.44 / 1.99
 //   192 x 64, Q = 32: 3,000 routes 0.89 / 0.92, 12,000 1.52 / 1.76
 //   192 x 64, Q = 72: 5,000 routes 2.07 / 1.99, 20,000 5.02 / 5.68, 57,000
 //     11.7 / 14.2; Q = 96: 2.53 / 2.43, 6.77 / 7.13, 16.5 / 17.8; 12,000 at
@@ -708,21 +712,27 @@ int exact_resident(Context* ctx, uint32_t lds)
 //     2.38, 12.5 / 11.5
 //   96 x 64, Q = 96: 12,000 4.43 / 3.84, 45,000 12.1 / 12.1; 128 x 48: 45,000
 //     12.0 / 11.0
-// (f16 rows, dim 512, Q = 416, 12 against 16 a CU: 12.4 / 10.9; f32 rows of 16 KB,
-// Q = 352, 6 against 7: 186 / 181.)
+// Float rows: narrow beams of launches that the spilling table holds (f32 dim
+// 640, Q = 224, 14 against 16 a CU: 1,800 rows a group 4.48 / 4.87, 14,800 rows 5.90 /
+// 5.48); f16 dim 512, Q = 416, 12 against 16: 12.4 / 10.9; f32 rows of 16 KB, Q = 352,
+// 6 against 7: 186 / 181.
 template <int kElem>
-bool slabs_cost(const Context* ctx, const ExactArgs& a, uint32_t count, int residents)
+bool spill_pays(const Context* ctx, const ExactArgs& a, uint32_t count, int spilling,
+                int residents)
 {
-    if (kElem != GOFANN_ELEM_U8) return false;
+    if (kElem != GOFANN_ELEM_U8)
+        return a.params.queue_limit <= narrow_beam(a.graph, 224, 160, 160) &&
+               all_resident(ctx, count, spilling);
+    if (a.params.queue_limit <= narrow_beam(a.graph, 160, 112, 64)) return true;
     const uint64_t round = static_cast<uint64_t>(residents) * static_cast<uint64_t>(ctx->compute_units);
-    if (a.params.queue_limit <= 72) return a.params.queue_limit <= 64 || count > round;
+    if (a.params.queue_limit <= 72) return count > round;
     return count > 2 * round && static_cast<uint64_t>(a.dim) * a.graph.degree >= 8192;
 }
 
 // Visited-set placement, then the launch.  Auto: the full LDS table where
 // full_table says so, else the most resident routes per CU, LDS preferred on
-// ties; where the slabs' traffic costs more than residents gain
-// (slabs_cost), the global slab has to hold more than a third more of them.
+// ties; where the spilling table pays (spill_pays), the global slab has to
+// hold more than a third more of them.
 // fixed_slab: visited slabs for a placement outside LDS, holding at most
 // fixed_routes routes (the no-alloc entry point); nullptr: context scratch.
 template <int kC, int kElem, int kR>
@@ -747,7 +757,7 @@ int launch_exact(Context* ctx, ExactArgs& a, int hash_mode, uint32_t lds_full,
                 mode = kVisitedSpill;
                 res = rs;
             }
-            if (rg > res + (slabs_cost<kElem>(ctx, a, count, rg) ? res / 3 : 0)) {
+            if (rg > res + (spill_pays<kElem>(ctx, a, count, rs, rg) ? res / 3 : 0)) {
                 mode = kVisitedGlobal;
                 res = rg;
             }

@@ -69,6 +69,12 @@ struct Context {
 // (registers, LDS and wave slots counted); 0 where none fits.
 int resident_blocks(Context* ctx, const void* kernel, uint32_t lds);
 
+// Whether every route of a launch is resident at `resident` a CU.
+inline bool all_resident(const Context* ctx, uint32_t routes, int resident)
+{
+    return static_cast<uint64_t>(resident) * static_cast<uint64_t>(ctx->compute_units) >= routes;
+}
+
 // Whether a launch of one wave64 per route keeps every visited set in a full LDS
 // table of its own (`lds` bytes a route, `resident` routes a CU), whatever
 // placement holds the most routes a CU: such routes run 3-7% faster, but their
@@ -86,9 +92,19 @@ int resident_blocks(Context* ctx, const void* kernel, uint32_t lds);
 inline bool full_table(const Context* ctx, uint32_t routes, uint32_t lds, int resident)
 {
     const uint64_t cus = static_cast<uint64_t>(ctx->compute_units);
-    if (static_cast<uint64_t>(resident) * cus < routes) return false;
+    if (!all_resident(ctx, routes, resident)) return false;
     return ctx->stream == nullptr ||
            (routes + cus - 1) / cus * lds <= static_cast<uint64_t>(ctx->lds_per_cu) / 4;
+}
+
+// The widest beam whose visited sets mostly stay well within the spilling table
+// (1,024 slots, probed in long runs past half of them): a set grows with the
+// beam and with the rows that a route can reach.  By rows a group: up to
+// 8,192, up to 16,384, more.
+inline int narrow_beam(const gofann_graph_view& g, int few, int some, int many)
+{
+    const uint32_t rows = g.groups > 0 ? g.rows / g.groups : g.rows;
+    return rows <= 8192 ? few : rows <= 16384 ? some : many;
 }
 
 int pq_search(Context* ctx, const gofann_pq_view* pq, const void* queries, int query_elem,

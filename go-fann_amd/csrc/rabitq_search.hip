@@ -101,7 +101,7 @@ int rabitq_search(Context* ctx, const gofann_rabitq_view* rq, const gofann_rabit
     if (rabitq_pair_eligible(rq, g, p))
         return rabitq_pair_search(ctx, make_rabitq_scorer(rq, pre), g, pred, r, p, out_ids,
                                   out_dists, stats);
-    const Placement pl = choose_visited<RabitqScorer>(ctx, l, p, r->count);
+    const Placement pl = choose_visited<RabitqScorer>(ctx, l, g, p, r->count);
     RabitqScorer sc = make_rabitq_scorer(rq, pre);
     // no neighbour past lane 31: rows scored a candidate per lane take two
     // lanes each (the whole-wave rows of 2048 / 4096 bits are unaffected)

@@ -1108,17 +1108,17 @@ struct Placement {
 // Visited-set placement for one scorer configuration.  hash_mode picks it;
 // auto takes the full LDS table where full_table says so (1,200 routes of 4096
 // bits: 7.63 ms, 7.90 with the global slab, 8.10 with the spilling table), the
-// spilling table where it holds the whole launch and the beam is narrow enough
-// for most sets to stay in it (32 subspaces, 3,900 routes, 16 a CU against 20 with
-// the slab: Q = 32 1.46 / 1.53 ms, Q = 64 2.22 / 2.28, Q = 80 2.60 / 2.65, Q = 128
-// 3.58 / 3.44; 9,000 routes, Q = 64 4.21 / 3.91), else the most resident routes
-// per CU, preferring LDS storage on ties (full table, then the spilling table,
+// spilling table where it holds the whole launch and the beam is narrow (32
+// subspaces, 16 a CU against 20 with the slab, 20,000 rows a group, 3,900 routes: Q =
+// 64 2.22 / 2.28 ms, Q = 80 2.60 / 2.65, Q = 128 3.58 / 3.44, and 9,000 routes at Q =
+// 64 4.21 / 3.91; 7,400 rows a group, 2,800 routes: Q = 96 1.99 / 2.05, Q = 128 2.57 /
+// 2.55, Q = 160 3.16 / 3.03; 1,800: Q = 128 2.16 / 2.30), else the most resident
+// routes per CU, preferring LDS storage on ties (full table, then the spilling table,
 // then the global slab).
 template <class Scorer>
-Placement choose_visited(Context* ctx, const Layout& l, const gofann_search_params* p,
-                         uint32_t routes)
+Placement choose_visited(Context* ctx, const Layout& l, const gofann_graph_view* g,
+                         const gofann_search_params* p, uint32_t routes)
 {
-    constexpr int kNarrow = 80;
     const int hash_mode = p->hash_mode;
     const auto at = [&](int visited, auto kern) {
         const int r = resident_per_cu(ctx, kern, l.bytes(visited));
@@ -1138,8 +1138,7 @@ Placement choose_visited(Context* ctx, const Layout& l, const gofann_search_para
         return pl;
     };
     if (full_table(ctx, routes, full.lds, full.resident)) return chosen(full);
-    if (p->queue_limit <= kNarrow && static_cast<uint64_t>(spill.resident) *
-                                             static_cast<uint64_t>(ctx->compute_units) >= routes)
+    if (p->queue_limit <= narrow_beam(*g, 128, 80, 80) && all_resident(ctx, routes, spill.resident))
         return chosen(spill);
     return best;
 }
@@ -1224,8 +1223,8 @@ int pq_search_ms(Context* ctx, const gofann_pq_view* pq, const void* queries, in
     const Layout ld = make_layout(DirectScorer::lds_bytes(pq->dim, pq->pq_dim), p->queue_limit,
                                   p->result_width);
     Placement pt{kVisitedGlobal, 0, 0, 0}, pd{kVisitedGlobal, 0, 0, 0};
-    if (p->table_mode != GOFANN_PLACE_GLOBAL) pt = choose_visited<TableScorer>(ctx, lt, p, r->count);
-    if (p->table_mode != GOFANN_PLACE_LDS) pd = choose_visited<DirectScorer>(ctx, ld, p, r->count);
+    if (p->table_mode != GOFANN_PLACE_GLOBAL) pt = choose_visited<TableScorer>(ctx, lt, g, p, r->count);
+    if (p->table_mode != GOFANN_PLACE_LDS) pd = choose_visited<DirectScorer>(ctx, ld, g, p, r->count);
     const bool direct = p->table_mode == GOFANN_PLACE_GLOBAL ||
                         (p->table_mode == GOFANN_PLACE_AUTO && pd.most > pt.most);
     ctx->last_table_in_lds = direct ? 0 : 1;

@@ -177,10 +177,10 @@ typedef struct {
      * into the global slab before it passes 3/4 load.
      * Auto: a launch whose routes are all resident with the table in LDS takes
      * it, on a stream other than the default one only up to a quarter of the
-     * LDS; other launches take the placement with the most resident routes per
-     * CU (narrow PQ and RaBitQ beams: the spilling table where it holds the
-     * whole launch; exact route, large u8 launches: the slab only if it holds
-     * over a third more than the spilling table). */
+     * LDS; a launch of narrow beams (narrower the more rows a group has) that
+     * the spilling table holds takes that; others take the placement with the
+     * most resident routes per CU (exact route, large u8 launches: the slab only
+     * if it holds over a third more than the spilling table). */
     int table_mode;
     int hash_mode;
 } gofann_search_params;

@@ -53,9 +53,11 @@ class Fake:
         self.hip.fake_clear()
         return out
 
+    group_rows = 100_000  # rows a group of the graphs
+
     def graph(self, degree=32):
         L, p = self.L, self.p
-        return L.GraphView(p, p, p, 1000, degree, 1, 1000, None)
+        return L.GraphView(p, p, p, 3 * self.group_rows, degree, 3, 1000, None)
 
     def routes(self, count):
         p = self.p
@@ -221,10 +223,18 @@ def case_narrow_beams_spill(f: Fake):
     takes it, though the slab would hold more (28)."""
     f.hip.fake_waves(28)
     h = f.context()
-    for beam, count, want in ((80, 21 * 256, "spill"), (81, 21 * 256, "global"),
-                              (80, 21 * 256 + 1, "global")):
+    for rows, beam, count, want in ((8193, 80, 21 * 256, "spill"), (8193, 81, 21 * 256, "global"),
+                                    (8192, 81, 21 * 256, "spill"), (8192, 129, 5000, "global"),
+                                    (8192, 80, 21 * 256 + 1, "global")):
+        f.group_rows = rows
         assert f.pq(h, 32, beam, count) == f.L.OK
-        assert f.placement(h)[1] == want, (beam, count)
+        assert f.placement(h)[1] == want, (rows, beam, count)
+    # exact f32 rows, dim 3072: 8 or 9 a CU against 10 or more; full table: 4
+    for rows, beam, want in ((8192, 224, "spill"), (8192, 225, "global"), (8193, 160, "spill"),
+                             (8193, 161, "global")):
+        f.group_rows = rows
+        assert f.exact(h, f.L.ELEM_F32, 3072, beam, 1500) == f.L.OK
+        assert f.placement(h)[1] == want, (rows, beam)
 
 
 def case_most_residents(f: Fake):
@@ -264,6 +274,12 @@ def case_u8_slabs(f: Fake):
             h, p, L.ELEM_U8, dim, 1000, p, f.graph(degree), None, L.PredicateView(),
             f.routes(count), L.ExactParams(beam, 1, 2, 0, 10, 0), p, p, None) == L.OK
         return f.placement(h)[1]
+    # narrow beams by the rows a group
+    for rows, beam, want in ((8192, 160, "spill"), (8192, 161, "global"), (16384, 112, "spill"),
+                             (16384, 113, "global"), (16385, 64, "spill"), (16385, 65, "global")):
+        f.group_rows = rows
+        assert placed(192, 32, beam, 4000) == want, (rows, beam)
+    f.group_rows = 100_000
     # (the rows' LDS pads the spilling table to 25 a CU)
     for dim, degree, beam, count, want in (
             (1088, 4, 64, 5000, "spill"), (1088, 8, 65, 5000, "global"),
